@@ -45,6 +45,7 @@ struct BatchView {
                      // periodic-1 kernels: 64; tiles of 32 and 128 run with the unroll of 4)
     double ewratio = 0.05;  // periodic 1: see pgrav_params.ewald_ratio
     int ngroups = 0;
+    int wave_slots = 8192;  // waves the GPU holds at 8 per SIMD
     int soft = 0;
     double eps = 0;
     double G = 1;

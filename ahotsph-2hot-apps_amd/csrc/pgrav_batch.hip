@@ -10,7 +10,8 @@
 //                          order-0 cells, bodies (u32 node / sorted-body slots)
 //   lpt    int[G]          groups by decreasing cost (longest first)
 //
-// Execution: one wave64 per group, one lane per sink (groups hold <= 64).
+// Execution: one lane per sink (groups hold <= 64), 4 to 16 wave64s per group, each
+// with an equal run of every list kind (split_log2); their sums meet in LDS.
 // A list is consumed in tiles of 64 entries: each lane fetches one entry's FP64
 // centre, subtracts the FP64 group centre, rounds the small offset to FP32 and
 // parks it in LDS; then every lane sweeps the tile, reading the offset as an
@@ -29,6 +30,8 @@
 #include "pgrav_ewald.h"
 
 namespace pgrav {
+
+constexpr int MAX_SPLIT = 16;  // waves that may share one group's lists
 
 template <typename T>
 struct V4 {
@@ -62,11 +65,20 @@ struct BatchArgs {
     double ewratio;      // periodic 1: expansion about the group centre when radius <= ewratio x distance
     int ngroups;
     int soft;
+    int lw;  // log2 of the waves that share a group's lists
     double eps;
     double G;
     double box;
     double ibox;  // 1 / box
 };
+
+// LDS traffic of one wave with itself: its LDS operations complete in order, so
+// only the compiler has to keep them on their side of this point.
+__device__ __forceinline__ void wave_sync() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
 
 // nearest periodic image of a displacement (identity when not periodic)
 template <bool PERIODIC, typename T>
@@ -93,6 +105,15 @@ struct EwShared {
     static constexpr int NP = PER == 1 ? 20 : 1;
     T part[NP][64];
     double acc[NP];
+    double trace;
+};
+
+// A wave's LDS: the staged tile, reused at a group's end for the wave's sums (64
+// entries), and its Ewald terms.
+template <typename T, int PER, int TILE>
+struct WaveShared {
+    V4<T> tile[TILE > 64 ? TILE : 64];
+    EwShared<T, PER> ew;
 };
 
 // The correction summed over a group's expanded sources (group radius small
@@ -228,13 +249,18 @@ __device__ __forceinline__ bool ewald_tile_entry(const BatchArgs &A, EwShared<T,
 // TILE: list entries staged in LDS per round (32, 64 or 128 -- one barrier pair and
 // one compensated fold per round; 64 in the periodic-1 kernels, whose per-entry
 // Ewald state is a lane's)
+// A group's 1 << A.lw waves (one workgroup) each take an equal run of every list
+// kind; the first wave adds their sums in wave order.
 template <typename T, bool REL, bool COMP, int SOFT, int PER, int BU, int TILE = 64>
-__device__ __forceinline__ void eval_group(const BatchArgs &A, int g, V4<T> *lds,
-                                           EwShared<T, PER> *ew) {
+__device__ __forceinline__ void eval_group(const BatchArgs &A, int g,
+                                           WaveShared<T, PER, TILE> *shared) {
     static_assert(TILE == 32 || TILE == 64 || TILE == 128, "tile of 32, 64 or 128 entries");
     static_assert(PER != 1 || TILE == 64, "the periodic-1 loader keeps one entry per lane");
     constexpr bool PERIODIC = PER == 1;
-    const int lane = threadIdx.x;
+    const int lane = threadIdx.x & 63;
+    const int w = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+    V4<T> *lds = shared[w].tile;
+    EwShared<T, PER> *ew = &shared[w].ew;
     const int cnt = A.gcount[g];
     const double4 gc = A.gcen[g];
     const bool live = lane < cnt;
@@ -274,7 +300,10 @@ __device__ __forceinline__ void eval_group(const BatchArgs &A, int g, V4<T> *lds
     for (int kind = 0; kind < 4; kind++) {
         const int64_t *offk = A.off + (int64_t)kind * (A.ngroups + 1);
         const uint32_t *__restrict__ idx = A.idx;
-        const int64_t o0 = offk[g], o1 = offk[g + 1];
+        // this wave's run of the list
+        const int64_t l0 = offk[g], l1 = offk[g + 1];
+        const int64_t share = (l1 - l0 + (1 << A.lw) - 1) >> A.lw;
+        const int64_t o0 = min(l1, l0 + w * share), o1 = min(l1, o0 + share);
         for (int64_t t0 = o0; t0 < o1; t0 += TILE) {
             const int nt = (int)min((int64_t)TILE, o1 - t0);
             uint64_t pmask = 0;  // periodic 1: bit k set when entry k takes the per-pair correction
@@ -305,7 +334,7 @@ __device__ __forceinline__ void eval_group(const BatchArgs &A, int g, V4<T> *lds
                     pmask = __builtin_amdgcn_ballot_w64(pair);
                 }
             }
-            __syncthreads();
+            wave_sync();
             Acc4T<T> p = {0, 0, 0, 0};
             // Offsets from the sink: an expanded source's image is the centre's for
             // every sink of the group (its offset from the centre was wrapped in the
@@ -368,19 +397,53 @@ __device__ __forceinline__ void eval_group(const BatchArgs &A, int g, V4<T> *lds
                 }
             }
 #undef PGRAV_OFFSET
-            __syncthreads();
+            wave_sync();
             fold<T>(s, c, p, COMP);
         }
     }
-    if (PERIODIC) {
-        // the lanes' running sums, summed per term in a fixed order (the last
-        // tile's barrier has passed)
-        if (lane < 20) {
-            double t = 0.0;
-            for (int k = 0; k < 64; k++) t += (double)ew->part[lane][k];
-            ew->acc[lane] = t;
+    if (A.lw) {
+        const double tr = PERIODIC ? wave_sum(trace) : 0.0;
+        if (w) {
+            lds[lane] = V4<T>{s.x, s.y, s.z, s.w};
+            if (PERIODIC && lane == 0)
+                ew->trace = tr;
         }
         __syncthreads();
+        if (!w)
+            for (int k = 1; k < (1 << A.lw); k++) {
+                const V4<T> q = shared[k].tile[lane];
+                fold<T>(s, c, Acc4T<T>{q.x, q.y, q.z, q.w}, COMP);
+                if (PERIODIC && lane == 0)
+                    trace += shared[k].ew.trace;
+            }
+        if (COMP) {
+            // the compensations follow through the same LDS
+            __syncthreads();
+            if (w)
+                lds[lane] = V4<T>{c.x, c.y, c.z, c.w};
+            __syncthreads();
+            if (!w)
+                for (int k = 1; k < (1 << A.lw); k++) {
+                    const V4<T> q = shared[k].tile[lane];
+                    c.x += q.x;
+                    c.y += q.y;
+                    c.z += q.z;
+                    c.w += q.w;
+                }
+        }
+        if (w)
+            return;
+    }
+    if (PERIODIC) {
+        // the lanes' running sums, summed per term in a fixed order
+        wave_sync();
+        if (lane < 20) {
+            double t = 0.0;
+            for (int v = 0; v < (1 << A.lw); v++)
+                for (int k = 0; k < 64; k++) t += (double)shared[v].ew.part[lane][k];
+            ew->acc[lane] = t;
+        }
+        wave_sync();
         Acc4T<T> p = {0, 0, 0, 0};
         // the expanded sources' correction at this sink's offset from the centre
         ewald_expansion_apply<T>(ew->acc, T(sp.x - gc.x), T(sp.y - gc.y), T(sp.z - gc.z), p);
@@ -424,11 +487,12 @@ struct MinWaves {
 
 // one workgroup per group, groups taken in longest-first order
 template <typename T, bool REL, bool COMP, int SOFT, int PER, int BU, int TILE>
-__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(MinWaves<T, PER, BU>::value)))
+__global__ __launch_bounds__(64 * MAX_SPLIT)
+__attribute__((amdgpu_waves_per_eu(MinWaves<T, PER, BU>::value)))
 void k_batch(BatchArgs A) {
-    __shared__ V4<T> lds[TILE];
-    __shared__ EwShared<T, PER> ew;
-    eval_group<T, REL, COMP, SOFT, PER, BU, TILE>(A, A.order_np[blockIdx.x], lds, &ew);
+    extern __shared__ __align__(16) char smem[];
+    eval_group<T, REL, COMP, SOFT, PER, BU, TILE>(A, A.order_np[blockIdx.x],
+                                                  (WaveShared<T, PER, TILE> *)smem);
 }
 
 // persistent: a fixed grid drains per-XCD work counters.  Workgroup b runs on
@@ -446,7 +510,8 @@ void k_batch(BatchArgs A) {
 // lists and records, and only pointers known to be distinct let the compiler
 // keep those reads on wave-uniform scalar loads.
 template <typename T, bool REL, bool COMP, int SOFT, int PER, int BU, int TILE>
-__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(MinWaves<T, PER, BU>::value)))
+__global__ __launch_bounds__(64 * MAX_SPLIT)
+__attribute__((amdgpu_waves_per_eu(MinWaves<T, PER, BU>::value)))
 void k_batch_persistent(
     BatchArgs A, const double4 *__restrict__ bpos, const double4 *__restrict__ cpos,
     const T *__restrict__ mom, const int64_t *__restrict__ gfirst, const int *__restrict__ gcount,
@@ -466,8 +531,7 @@ void k_batch_persistent(
     A.out = out;
     A.counter = counter;
     A.ewald = ewald;
-    __shared__ V4<T> lds[TILE];
-    __shared__ EwShared<T, PER> ew;
+    extern __shared__ __align__(16) char smem[];
     __shared__ int w;
     const int x = blockIdx.x % NXCD;
     // own slice first; once it is drained, the next group of the other XCDs' slices
@@ -494,7 +558,8 @@ void k_batch_persistent(
         __syncthreads();
         if (item < 0)
             break;
-        eval_group<T, REL, COMP, SOFT, PER, BU, TILE>(A, A.lpt[item], lds, &ew);
+        eval_group<T, REL, COMP, SOFT, PER, BU, TILE>(A, A.lpt[item],
+                                                      (WaveShared<T, PER, TILE> *)smem);
     }
     if (threadIdx.x == 0) {
         const int done = atomicAdd(&A.counter[1], 1);
@@ -508,9 +573,8 @@ void k_batch_persistent(
 // the FP64 "plain" reference dispatch: one launch per group (nln/pgrav.cu:1078)
 template <int SOFT, int PER>
 __global__ __launch_bounds__(64) void k_group64(BatchArgs A, int g) {
-    __shared__ V4<double> lds[64];
-    __shared__ EwShared<double, PER> ew;
-    eval_group<double, false, false, SOFT, PER, 4>(A, g, lds, &ew);
+    __shared__ WaveShared<double, PER, 64> shared[1];
+    eval_group<double, false, false, SOFT, PER, 4>(A, g, shared);
 }
 
 __global__ void k_reset_counter(int *c) {
@@ -721,18 +785,45 @@ hipError_t launch_reset_counter(int *c, hipStream_t st) {
     return hipGetLastError();
 }
 
+// Waves that share one group's lists, as a power of two.  A group's lists are a
+// serial chain of LDS tiles and scalar record loads: a wave alone on its SIMD runs
+// at its latency (1 us per order-4 cell), and a launch of a few groups per wave slot
+// ends in a tail of long lists.  Four waves cost nothing where there are many groups;
+// eight and sixteen pay while the groups are few.  us per evaluation by 1, 2, 4, 8, 16
+// waves a group (order 4, theta 0.6 unless stated; in brackets: passes of two plans in
+// turn on two streams, where the tails overlap):
+//   111 groups (Plummer 4,099)            985   486   241   124    65
+//   1,469 (Plummer 65,536, order 2)      1049   525   280   178   143
+//   4,100 (lattice 64^3, images)         2054  1332  1176  1150  1139 [1713 .. 1051 1061 1073]
+//   4,110 (clustered 262,144, FP64)      2217  1735  1367  1281  1348 [1572 .. 1166 1173 1267]
+//   16,457 (clustered 1 M, tolerance)    2012  1613  1333  1246  1300 [1399 .. 1165 1151 1229]
+//   25,034 (clustered 1 M)               3247  2895  2591  2527  2678 [2605 .. 2401 2421 2585]
+//   32,795 (lattice 128^3, Ewald)        5562  5167  4956  5130  5121 [4928 .. 4779 5027 5037]
+//   263,505 (clustered 16.8 M), ms       42.4  42.0  41.2  41.6  44.0 [40.5 .. 40.3 41.9 45.2]
+static int split_log2(int ngroups, int wave_slots) {
+    if (ngroups < wave_slots / 2)
+        return 4;
+    return ngroups < 4 * wave_slots ? 3 : 2;
+}
+
 template <typename T, bool REL, bool COMP, int SOFT, int PER, int BU, int TILE = 64>
-static void launch_one(const BatchArgs &A, int persistent_blocks, hipStream_t st) {
-    // every XCD needs workgroups to drain its slice: round up to a multiple of NXCD
-    persistent_blocks = (persistent_blocks + NXCD - 1) / NXCD * NXCD;
-    if (persistent_blocks > 0)
-        hipLaunchKernelGGL((k_batch_persistent<T, REL, COMP, SOFT, PER, BU, TILE>),
-                           dim3(persistent_blocks), dim3(64), 0, st, A, A.bpos, A.cpos,
-                           (const T *)A.mom, A.gfirst, A.gcount, A.gcen, A.lpt, A.xoff, A.off,
-                           A.idx, (V4<T> *)A.out, A.counter, A.ewald);
-    else
-        hipLaunchKernelGGL((k_batch<T, REL, COMP, SOFT, PER, BU, TILE>), dim3(A.ngroups), dim3(64),
-                           0, st, A);
+static void launch_one(BatchArgs A, int persistent_blocks, hipStream_t st) {
+    // a workgroup's LDS stays within 64 KB (the Ewald terms take 5 or 10 KB a wave)
+    while (A.lw && (sizeof(WaveShared<T, PER, TILE>) << A.lw) > 65536) A.lw--;
+    const int waves = 1 << A.lw;
+    const unsigned lds = (unsigned)(waves * sizeof(WaveShared<T, PER, TILE>));
+    if (persistent_blocks > 0) {
+        // persistent_blocks counts waves; every XCD needs workgroups to drain its slice,
+        // so round up to a multiple of NXCD
+        const int grid = ((persistent_blocks + waves - 1) / waves + NXCD - 1) / NXCD * NXCD;
+        hipLaunchKernelGGL((k_batch_persistent<T, REL, COMP, SOFT, PER, BU, TILE>), dim3(grid),
+                           dim3(64 * waves), lds, st, A, A.bpos, A.cpos, (const T *)A.mom, A.gfirst,
+                           A.gcount, A.gcen, A.lpt, A.xoff, A.off, A.idx, (V4<T> *)A.out,
+                           A.counter, A.ewald);
+    } else {
+        hipLaunchKernelGGL((k_batch<T, REL, COMP, SOFT, PER, BU, TILE>), dim3(A.ngroups),
+                           dim3(64 * waves), lds, st, A);
+    }
 }
 
 // the unroll factor and the tile: choices for the group-relative compensated FP32
@@ -803,6 +894,7 @@ hipError_t launch_batch(const BatchView &v, int variant, int persistent_blocks, 
     A.unroll = v.unroll;
     A.tile = v.tile;
     A.ewratio = v.ewratio;
+    A.lw = split_log2(v.ngroups, v.wave_slots);
     if (A.ngroups <= 0)
         return hipSuccess;
     if (v.periodic < 0 || v.periodic > 2 || (v.periodic == 2 && !v.img))
@@ -848,6 +940,7 @@ hipError_t launch_group64(const BatchView &v, int g, hipStream_t st) {
     A.unroll = v.unroll;
     A.tile = v.tile;
     A.ewratio = v.ewratio;
+    A.lw = 0;
     if (v.periodic < 0 || v.periodic > 2 || (v.periodic == 2 && !v.img))
         return hipErrorInvalidValue;
     const int per = v.periodic;

@@ -142,14 +142,13 @@ void Plan::ensure_moments_view() {
     mv.mom64 = (double *)v.mom64;
 }
 
-static int auto_blocks() {
+// waves that fill the current device: 32 per CU, 8 per SIMD
+static int device_wave_slots() {
     int dev = 0, cus = 256;
-    if (hipGetDevice(&dev) == hipSuccess) {
-        hipDeviceProp_t pr;
-        if (hipGetDeviceProperties(&pr, dev) == hipSuccess)
-            cus = pr.multiProcessorCount;
-    }
-    return cus * 32;  // 32 single-wave workgroups per CU: 8 per SIMD, a full CU
+    if (hipGetDevice(&dev) != hipSuccess ||
+        hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess)
+        cus = 256;
+    return cus * 32;
 }
 
 static hipStream_t stream_of(Plan *P, void *stream) {
@@ -254,7 +253,7 @@ static int evaluate(Plan *P, int variant, hipStream_t st) {
     }
     int pb = P->prm.persistent_blocks;
     if (pb < 0)
-        pb = auto_blocks();
+        pb = P->v.wave_slots;
     if (!check(launch_batch(P->v, variant, pb, st), "batched kernel"))
         return -1;
     return far_field(P, variant, st);
@@ -378,6 +377,7 @@ void *pgrav_plan_create(const double *pos3, const double *mass, int64_t n, const
         // groups and lists
         Lists &L = P->lists;
         P->v.ngroups = (int)L.ngroups;
+        P->v.wave_slots = device_wave_slots();
         P->v.gfirst = P->upload(L.gfirst.data(), L.gfirst.size());
         P->v.gcount = P->upload(L.gcount.data(), L.gcount.size());
         if (!L.gslots.empty()) {

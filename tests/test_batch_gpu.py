@@ -268,3 +268,24 @@ def test_plan_rejects_bad_input(gpu_lib):
         batch.Plan(pos, np.full(100, 0.01), soft="plummer", eps=0.0)
     with pytest.raises(PgravError):
         batch.Plan(pos, np.full(100, 0.01), soft=3)
+
+
+@pytest.mark.parametrize("n", [2, 65, 4095, 4096, 32767, 32768])
+def test_shared_lists_match_oracle(setup, n):
+    """Lists shared by 16, 8 or 4 waves of a workgroup, by the number of groups
+    (one-body groups here: n of them, at each side of the rule's steps on 256 CUs),
+    some lists shorter than the waves: FP32 and FP64 against the oracle's FP64
+    evaluation of the same lists, and one launch shape bit for bit as the other."""
+    batch, ics, _, _ = setup
+    pos, mass = ics.clustered(n, seed=5, nhalo=8)
+    kw = dict(theta=1.0, order=2, eps=1e-3, group_max=1, leaf_max=4, merge_groups=0)
+    e = _group_errors(batch, pos, mass, kw, ["rel32c", "f64"], ngroups=min(n, 12))
+    # FP32 offsets and a few hundred terms per sink, as above
+    assert e["f64"] < 1e-10 and e["rel32c"] < 1e-5, e
+    plan = batch.Plan(pos, mass, **kw)
+    plan.evaluate("rel32c")
+    want = plan.result("rel32c")
+    plan.set_launch(0)
+    plan.evaluate("rel32c")
+    np.testing.assert_array_equal(plan.result("rel32c"), want)
+    plan.close()

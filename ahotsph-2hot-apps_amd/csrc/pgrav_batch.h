@@ -38,6 +38,13 @@ struct BatchView {
     float4 *out32 = nullptr;
     double4 *out64 = nullptr;
     int *counter = nullptr;
+    double *far2 = nullptr;  // per group: square of its far distance (k_far); null: no expansions
+    float4 *far_lo = nullptr;  // the far cells' pull: out32 and this remainder
+    // the cell entries (and images) the expansions leave to the pair kernels, each list from
+    // its own start in idx, and their number [3][ngroups]
+    uint32_t *near = nullptr;
+    uint8_t *near_img = nullptr;
+    int *near_n = nullptr;
     const float *ewald32 = nullptr;   // Ewald correction table (pgrav_ewald.h), FP32 copy
     const double *ewald64 = nullptr;  // FP64
     int unroll = 4;  // order-0 / body loop unroll of the rel32c kernels: 2, 4 or 8
@@ -55,6 +62,8 @@ struct BatchView {
 };
 
 hipError_t launch_batch(const BatchView &v, int variant, int persistent_blocks, hipStream_t st);
+// the far cells' pull into out32 and the groups' far distances into far2 (pgrav_far.hip)
+hipError_t launch_far(const BatchView &v, hipStream_t st);
 hipError_t launch_group64(const BatchView &v, int g, hipStream_t st);
 hipError_t launch_reset_counter(int *c, hipStream_t st);
 hipError_t launch_ewald_table(double L, double *t64, float *t32, hipStream_t st);

@@ -28,6 +28,7 @@
 #include "pgrav_batch.h"
 #include "pgrav_device.h"
 #include "pgrav_ewald.h"
+#include "pgrav_far.h"
 
 namespace pgrav {
 
@@ -62,6 +63,12 @@ struct BatchArgs {
     int img_f;           // 2 nimage + 1 images per side
     int unroll;          // order-0 / body loop unroll of the rel32c kernels: 2, 4 or 8
     int tile;            // list entries staged in LDS per round (rel32c, not periodic 1): 32, 64, 128
+    const double *far2;  // per group: square of its far distance (null: no expansions)
+    const float4 *far_lo;  // the far cells' pull: out and this remainder
+    // what the expansion leaves of the cell lists (periodic 1: the kernel decides itself)
+    const uint32_t *near;
+    const uint8_t *near_img;
+    const int *near_n;
     double ewratio;      // periodic 1: expansion about the group centre when radius <= ewratio x distance
     int ngroups;
     int soft;
@@ -71,14 +78,6 @@ struct BatchArgs {
     double box;
     double ibox;  // 1 / box
 };
-
-// LDS traffic of one wave with itself: its LDS operations complete in order, so
-// only the compiler has to keep them on their side of this point.
-__device__ __forceinline__ void wave_sync() {
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-}
 
 // nearest periodic image of a displacement (identity when not periodic)
 template <bool PERIODIC, typename T>
@@ -163,28 +162,15 @@ __device__ __forceinline__ void fold(Acc4T<T> &s, Acc4T<T> &c, const Acc4T<T> &p
     }
 }
 
-// Group-relative (REL) or absolute offset of a source centre, rounded to T.
+// Group-relative (REL) or absolute offset of a source centre, rounded to T; d is its
+// FP64 offset from the group centre.
 template <typename T, bool REL, bool PERIODIC>
-__device__ __forceinline__ V4<T> source_offset(double4 c, double4 gc, double box, double ibox) {
-    double dx = c.x, dy = c.y, dz = c.z;
-    if (REL || PERIODIC) {
-        dx -= gc.x;
-        dy -= gc.y;
-        dz -= gc.z;
-    }
-    if (PERIODIC) {
-        // (a product with 1 / box, not a division: the image of a source exactly half
-        // a box away is a tie either way)
-        dx -= box * rint(dx * ibox);
-        dy -= box * rint(dy * ibox);
-        dz -= box * rint(dz * ibox);
-        if (!REL) {  // absolute variant: re-add the group centre after wrapping
-            dx += gc.x;
-            dy += gc.y;
-            dz += gc.z;
-        }
-    }
-    return V4<T>{T(dx), T(dy), T(dz), T(c.w)};
+__device__ __forceinline__ V4<T> source_offset(double4 c, double3 d, double4 gc) {
+    if (REL)
+        return V4<T>{T(d.x), T(d.y), T(d.z), T(c.w)};
+    if (PERIODIC)  // absolute: the image nearest the group centre
+        return V4<T>{T(d.x + gc.x), T(d.y + gc.y), T(d.z + gc.z), T(c.w)};
+    return V4<T>{T(c.x), T(c.y), T(c.z), T(c.w)};
 }
 
 // The Ewald correction of one tile entry (periodic = 1), in the tile loader:
@@ -194,26 +180,19 @@ __device__ __forceinline__ V4<T> source_offset(double4 c, double4 gc, double box
 // lane holds an entry; the terms go to the lane's own running sums in LDS.
 template <typename T, int PER>
 __device__ __forceinline__ bool ewald_tile_entry(const BatchArgs &A, EwShared<T, PER> *ew, bool on,
-                                                 int lane, double4 src, double4 gc, bool cell,
-                                                 const T *rec) {
+                                                 int lane, double mass, double3 d, double4 gc,
+                                                 bool cell, const T *rec) {
     T v[20];
     bool pair = false;
     if (on) {
-        double dx = src.x - gc.x, dy = src.y - gc.y, dz = src.z - gc.z;
-        dx -= A.box * rint(dx * A.ibox);
-        dy -= A.box * rint(dy * A.ibox);
-        dz -= A.box * rint(dz * A.ibox);
-        const double am = fmax(fabs(dx), fmax(fabs(dy), fabs(dz)));
-        // the expansion holds when every sink sees the centre's image of the source
-        // and the source's other images are far against the group radius
-        const bool expand = am < 0.5 * A.box - gc.w && gc.w <= A.ewratio * (A.box - am);
+        const bool expand = ewald_expands(d, gc, A.box, A.ewratio);
         pair = !expand;
 #pragma unroll
         for (int q = 0; q < 20; q++) v[q] = T(0);
         if (expand) {
             EwField<T> F;
-            ewald_field<T>(ewald_table(A, T(0)), T(dx), T(dy), T(dz), T(A.box), F);
-            const T m = T(src.w);
+            ewald_field<T>(ewald_table(A, T(0)), T(d.x), T(d.y), T(d.z), T(A.box), F);
+            const T m = T(mass);
             v[0] = m * F.psi;
 #pragma unroll
             for (int q = 0; q < 3; q++) v[1 + q] = m * F.c[q];
@@ -257,6 +236,8 @@ __device__ __forceinline__ void eval_group(const BatchArgs &A, int g,
     static_assert(TILE == 32 || TILE == 64 || TILE == 128, "tile of 32, 64 or 128 entries");
     static_assert(PER != 1 || TILE == 64, "the periodic-1 loader keeps one entry per lane");
     constexpr bool PERIODIC = PER == 1;
+    // the group-relative FP32 kernels leave the far cells to the group's expansion
+    constexpr bool FAR = REL && sizeof(T) == 4;
     const int lane = threadIdx.x & 63;
     const int w = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
     V4<T> *lds = shared[w].tile;
@@ -288,6 +269,18 @@ __device__ __forceinline__ void eval_group(const BatchArgs &A, int g,
     const T ibox = T(1) / box;
     const T *__restrict__ mom = (const T *)A.mom;
     Acc4T<T> s = {0, 0, 0, 0}, c = {0, 0, 0, 0};
+    double far2 = INFINITY;
+    if constexpr (FAR) {
+        if (A.far2)
+            far2 = A.far2[g];
+        if (far2 < (double)INFINITY && w == 0) {  // the far cells' pull at this sink (k_far)
+            const V4<T> f = ((const V4<T> *)A.out)[slot];
+            const float4 lo = A.far_lo[slot];
+            s = Acc4T<T>{f.x, f.y, f.z, f.w};
+            if (COMP)
+                c = Acc4T<T>{lo.x, lo.y, lo.z, lo.w};
+        }
+    }
     // periodic: this lane's share of the listed cells' second-moment traces (the
     // potential's second-order Ewald term, the same for every sink of the group)
     double trace = 0.0;
@@ -299,39 +292,45 @@ __device__ __forceinline__ void eval_group(const BatchArgs &A, int g,
 #pragma unroll 1
     for (int kind = 0; kind < 4; kind++) {
         const int64_t *offk = A.off + (int64_t)kind * (A.ngroups + 1);
-        const uint32_t *__restrict__ idx = A.idx;
+        const bool left = FAR && PER != 1 && kind < 3 && far2 < (double)INFINITY;
+        const uint32_t *__restrict__ idx = left ? A.near : A.idx;
+        const uint8_t *__restrict__ img = left ? A.near_img : A.img;
+        // the entry a whole wave takes: a scalar load (nothing writes lists in this launch)
+        const auto *cidx = (const __attribute__((address_space(4))) uint32_t *)idx;
         // this wave's run of the list
-        const int64_t l0 = offk[g], l1 = offk[g + 1];
+        const int64_t l0 = offk[g], l1 = left ? l0 + A.near_n[kind * A.ngroups + g] : offk[g + 1];
         const int64_t share = (l1 - l0 + (1 << A.lw) - 1) >> A.lw;
         const int64_t o0 = min(l1, l0 + w * share), o1 = min(l1, o0 + share);
         for (int64_t t0 = o0; t0 < o1; t0 += TILE) {
             const int nt = (int)min((int64_t)TILE, o1 - t0);
             uint64_t pmask = 0;  // periodic 1: bit k set when entry k takes the per-pair correction
+            uint64_t near = 0;   // and when it is taken in pairs
 #pragma unroll
             for (int h = 0; h < (TILE + 63) / 64; h++) {
                 const int u = lane + 64 * h;  // the tile entry this lane loads
-                double4 src = make_double4(0, 0, 0, 0);
+                double mass = 0;
+                double3 d = make_double3(0, 0, 0);
                 uint32_t e = 0;
+                bool far = false;
                 if (u < nt) {
                     e = idx[t0 + u];
-                    src = kind == 3 ? A.bpos[e] : A.cpos[e];
-                    if (PER == 2) {
-                        // image (i, j, k) in nln/mac.c:91-111 order: the source sits at
-                        // x + (i, j, k) box, added in FP64
-                        const int im = A.img[t0 + u], f = A.img_f, hf = f >> 1;
-                        src.x += (double)(im / (f * f) - hf) * A.box;
-                        src.y += (double)((im / f) % f - hf) * A.box;
-                        src.z += (double)(im % f - hf) * A.box;
-                    }
-                    lds[u] = source_offset<T, REL, PERIODIC>(src, gc, A.box, A.ibox);
-                    if (PERIODIC && kind < 3)
+                    const double4 src = entry_position<PER>(kind == 3 ? A.bpos : A.cpos, e, img,
+                                                            t0 + u, A.img_f, A.box);
+                    d = entry_offset<PER>(src, gc, A.box, A.ibox);
+                    mass = src.w;
+                    lds[u] = source_offset<T, REL, PERIODIC>(src, d, gc);
+                    if (PERIODIC && kind < 3) {
                         trace += (double)mom[(size_t)e * PREC4 + PREC_TRACE];
+                        far = FAR && offk[g + 1] - offk[g] >= FAR_MIN_LIST &&
+                              entry_far<PER>(d, far2, gc, A.box, A.ewratio);
+                    }
                 }
                 if (PERIODIC) {
-                    const bool pair = ewald_tile_entry<T, PER>(A, ew, u < nt, lane, src, gc,
+                    const bool pair = ewald_tile_entry<T, PER>(A, ew, u < nt, lane, mass, d, gc,
                                                                kind < 3, mom + (size_t)e * PREC4);
-                    // one entry per lane (TILE 64): the wave's flags as a scalar mask
+                    // one entry per lane (TILE 64): the wave's flags as scalar masks
                     pmask = __builtin_amdgcn_ballot_w64(pair);
+                    near = __builtin_amdgcn_ballot_w64(u < nt && !far);
                 }
             }
             wave_sync();
@@ -348,9 +347,24 @@ __device__ __forceinline__ void eval_group(const BatchArgs &A, int g,
         y = pbc<PERIODIC>(y, box, ibox);                            \
         z = pbc<PERIODIC>(z, box, ibox);                            \
     }
-            if (kind == 0) {
+            if (FAR && PER == 1 && kind < 3) {
+                for (; near; near &= near - 1) {
+                    const int k = __builtin_ctzll(near);
+                    const uint32_t ek = cidx[t0 + k];
+                    const V4<T> r = lds[k];
+                    PGRAV_OFFSET(r, x, y, z, pp)
+                    if (kind == 0)
+                        cell_interact<4, false, 1, T>(mom + (size_t)ek * PREC4, r.w, x, y, z, eps2_cell, p);
+                    else if (kind == 1)
+                        cell_interact<2, false, 1, T>(mom + (size_t)ek * PREC4, r.w, x, y, z, eps2_cell, p);
+                    else
+                        mono_interact<T>(r.w, x, y, z, eps2_cell, p);
+                    if (pp)
+                        ewald_pair<T>(ewald_table(A, T(0)), r.w, x, y, z, box, p);
+                }
+            } else if (kind == 0) {
                 for (int k = 0; k < nt; k++) {
-                    const uint32_t ek = idx[t0 + k];
+                    const uint32_t ek = cidx[t0 + k];
                     const V4<T> r = lds[k];
                     PGRAV_OFFSET(r, x, y, z, pp)
                     cell_interact<4, false, 1, T>(mom + (size_t)ek * PREC4, r.w, x, y, z, eps2_cell, p);
@@ -359,7 +373,7 @@ __device__ __forceinline__ void eval_group(const BatchArgs &A, int g,
                 }
             } else if (kind == 1) {
                 for (int k = 0; k < nt; k++) {
-                    const uint32_t ek = idx[t0 + k];
+                    const uint32_t ek = cidx[t0 + k];
                     const V4<T> r = lds[k];
                     PGRAV_OFFSET(r, x, y, z, pp)
                     cell_interact<2, false, 1, T>(mom + (size_t)ek * PREC4, r.w, x, y, z, eps2_cell, p);
@@ -894,6 +908,21 @@ hipError_t launch_batch(const BatchView &v, int variant, int persistent_blocks, 
     A.unroll = v.unroll;
     A.tile = v.tile;
     A.ewratio = v.ewratio;
+    A.far2 = nullptr;
+    A.far_lo = nullptr;
+    A.near = nullptr;
+    A.near_img = nullptr;
+    A.near_n = nullptr;
+    if ((variant == VAR_REL32C || variant == VAR_REL32) && v.far2) {
+        A.far2 = v.far2;
+        A.far_lo = v.far_lo;
+        A.near = v.near;
+        A.near_img = v.near_img;
+        A.near_n = v.near_n;
+        const hipError_t e = launch_far(v, st);
+        if (e != hipSuccess)
+            return e;
+    }
     A.lw = split_log2(v.ngroups, v.wave_slots);
     if (A.ngroups <= 0)
         return hipSuccess;
@@ -940,6 +969,11 @@ hipError_t launch_group64(const BatchView &v, int g, hipStream_t st) {
     A.unroll = v.unroll;
     A.tile = v.tile;
     A.ewratio = v.ewratio;
+    A.far2 = nullptr;
+    A.far_lo = nullptr;
+    A.near = nullptr;
+    A.near_img = nullptr;
+    A.near_n = nullptr;
     A.lw = 0;
     if (v.periodic < 0 || v.periodic > 2 || (v.periodic == 2 && !v.img))
         return hipErrorInvalidValue;

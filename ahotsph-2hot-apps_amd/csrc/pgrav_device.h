@@ -183,6 +183,14 @@ __device__ __forceinline__ void k1_interact(T m, T x, T y, T z, T eps_inv, T eps
     a.z += z * eqe;
 }
 
+// LDS traffic of one wave with itself: its LDS operations complete in order, so
+// only the compiler has to keep them on their side of this point.
+__device__ __forceinline__ void wave_sync() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
 // ---------------------------------------------------------------- wave sums
 // The sum of a value over the 64 lanes of a wave by DPP row operations (VALU
 // only, no LDS): pairs and quads by quad permutes, 8 and 16 lanes by the half-

@@ -151,6 +151,28 @@ static int device_wave_slots() {
     return cus * 32;
 }
 
+// Whether the FP32 kernels take far cells through local expansions (pgrav_far.hip).
+// By the lists' mean: the expansion saves ~38 VALU instructions a wave for every
+// order-4 cell listed and ~8 for an order-2 cell, nothing worth it for an order-0 cell
+// (16 instructions in a pair), and costs ~6,500 a group; the launch and its serial
+// chain cost ~35 us, 4,000 instructions per wave slot.  The Ewald kernel still reads
+// every entry for the correction and gains only with many groups.  us per evaluation in
+// pairs and with expansions (groups, cells listed by each):
+//   clustered 65,536 (1,830, 269)     172  177    Plummer 65,536 (1,452, 667)   283  302
+//   clustered 131,072 (3,679, 353)    340  308    Plummer 262,144 (5,738, 943)  907  668
+//   clustered 524,288 (14,061, 506)  1283 1032    clustered 2 M (32,903, 748)  4500 3555
+//   images 32^3 (512, 1,600)          204  200    images 64^3 (4,102, 1,908)   1197  810
+//   order 2, 1 M (26,465, 773)       1357 1412    order 2 Plummer 262,144 (5,738, 1,109) 479 452
+//   order 0, 1 M (26,465, 813)        870  945    tolerance 1 M (16,454, 47 + 22 + 1,704) 1272 1378
+//   Ewald 64^3 (4,102, 794)          1241 1294    Ewald 96^3 (16,384, 794) 3617 3387
+//   Ewald 128^3 (32,795, 910)        5281 4014
+static bool far_pays(const Lists &L, int wave_slots, int periodic) {
+    const int64_t G = L.ngroups;
+    return 38 * L.off[L_HEXA].back() + 8 * L.off[L_QUAD].back() >
+               6500 * G + (int64_t)4000 * wave_slots &&
+           (periodic != 1 || G >= 2 * (int64_t)wave_slots);
+}
+
 static hipStream_t stream_of(Plan *P, void *stream) {
     return stream ? (hipStream_t)stream : P->stream;
 }
@@ -427,6 +449,18 @@ void *pgrav_plan_create(const double *pos3, const double *mass, int64_t n, const
         P->v.out32 = P->dalloc<float4>(sizeof(float4) * (size_t)n);
         if (p->fp64)
             P->v.out64 = P->dalloc<double4>(sizeof(double4) * (size_t)n);
+        if (far_pays(L, P->v.wave_slots, p->periodic)) {
+            // the local expansions' workspace: the far cells' pull and the rest of the lists
+            const size_t G = std::max(1, P->v.ngroups);
+            int64_t cells = 0;
+            for (int k = 0; k < L_BODY; k++) cells += L.off[k].back();
+            P->v.far2 = P->dalloc<double>(sizeof(double) * G);
+            P->v.far_lo = P->dalloc<float4>(sizeof(float4) * (size_t)n);
+            P->v.near_n = P->dalloc<int>(sizeof(int) * 3 * G);
+            P->v.near = P->dalloc<uint32_t>(sizeof(uint32_t) * cells);
+            if (p->periodic == 2)
+                P->v.near_img = P->dalloc<uint8_t>(cells);
+        }
         P->v.counter = P->dalloc<int>(64);
         if (!check(hipMemset(P->v.counter, 0, 64), "hipMemset"))
             throw std::runtime_error("memset");

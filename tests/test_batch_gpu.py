@@ -289,3 +289,62 @@ def test_shared_lists_match_oracle(setup, n):
     plan.evaluate("rel32c")
     np.testing.assert_array_equal(plan.result("rel32c"), want)
     plan.close()
+
+
+def _far_pays(st, ewald):
+    # the rule of pgrav_plan.hip for 256 CUs (the Ewald kernel's too)
+    return 38 * st["entries_hexa"] + 8 * st["entries_quad"] > 6500 * st["ngroups"] + 4000 * 8192 \
+        and (not ewald or st["ngroups"] >= 2 * 8192)
+
+
+@pytest.mark.parametrize("kw", [
+    dict(order=4, soft="plummer", eps=1e-3, merge_groups=1),
+    dict(order=4, soft="plummer", eps=1e-3, merge_groups=5, rcb_cell=4096),
+    dict(order=4, soft="none", eps=0.0, merge_groups=1),
+    dict(order=4, soft="k1", eps=2e-3, merge_groups=1),
+    dict(order=2, theta=0.3, soft="plummer", eps=1e-3, merge_groups=1),
+    dict(order=4, soft="plummer", eps=1e-3, mac="tolerance", errtol=5e-4, quad_ncut=10,
+         hexa_ncut=10, leaf_max=8),
+    dict(order=4, theta=0.4, soft="plummer", eps=1e-3, periodic="images", nimage=1, box=1.0),
+    dict(order=4, soft="plummer", eps=1e-3, periodic="ewald", box=1.0, group_max=4),
+], ids=["plummer", "bisection", "unsoftened", "k1", "order2", "tolerance", "images", "ewald"])
+def test_far_cells_match_the_pairs(gpu_lib, kw):
+    """Plans whose far cells go through local expansions: FP32 against the batched FP64
+    evaluation of the same lists (which takes every cell in pairs), on the plan's bodies
+    and after they moved by a few group radii, where the far distance has to follow; and
+    bit for bit the same from a graph and from either launch shape."""
+    from pgrav import batch, ics
+    pos, mass = ics.clustered(60000, seed=21, nhalo=24)
+    pos = (pos - pos.min(0)) / (np.ptp(pos, 0).max() * 1.001)
+    kw = dict(dict(theta=0.6, group_max=8, leaf_max=16), **kw)
+    plan = batch.Plan(pos, mass, **kw)
+    assert _far_pays(plan.stats(), kw.get("periodic") == "ewald"), plan.stats()
+    rng = np.random.default_rng(3)
+    for move in (0.0, 1e-3):
+        if move:
+            plan.update(pos + rng.normal(0, move, pos.shape), mass)
+        plan.evaluate("f64")
+        ref = plan.result("f64")
+        for var in ("rel32c", "rel32"):
+            plan.evaluate(var)
+            got = plan.result(var)
+            # an FP32 pair kernel's error: a few 1e-7 of the pulls' sum, which the
+            # periodic images' partial cancellation raises against the result
+            da = np.linalg.norm(got[:, :3] - ref[:, :3], axis=1)
+            scale = np.linalg.norm(ref[:, :3], axis=1) + np.median(np.linalg.norm(ref[:, :3], axis=1))
+            dp = np.abs(got[:, 3] - ref[:, 3]) / np.median(np.abs(ref[:, 3]))
+            tol = 3e-5 if kw.get("periodic") else 3e-6
+            assert np.percentile(da / scale, 99) < tol and np.percentile(dp, 99) < tol, \
+                (var, move, np.percentile(da / scale, [50, 99, 100]), dp.max())
+    plan.evaluate("rel32c")
+    want = plan.result("rel32c")
+    plan.set_launch(0)
+    plan.evaluate("rel32c")
+    np.testing.assert_array_equal(plan.result("rel32c"), want)
+    plan.graph_capture("rel32c")
+    for _ in range(3):
+        plan.evaluate("f64")
+        plan.synchronize()
+        plan.graph_launch()
+        np.testing.assert_array_equal(plan.result("rel32c"), want)
+    plan.close()

@@ -348,3 +348,18 @@ def test_far_cells_match_the_pairs(gpu_lib, kw):
         plan.graph_launch()
         np.testing.assert_array_equal(plan.result("rel32c"), want)
     plan.close()
+
+
+@pytest.mark.parametrize("ns", [1, 15, 16, 17, 65, 1025])
+def test_direct_sum_sample_sizes(setup, ns):
+    """The FP64 direct sum for samples around the sizes of its blocks (16 sinks summed
+    per workgroup, 64 evaluated), against the oracle: each of n = 40,000 terms carries a
+    few rounding errors of 2^-53 and the sums' are below n 2^-53 of the summed pulls."""
+    batch, ics, pos, mass = setup
+    plan = batch.Plan(pos, mass, theta=0.8, order=0, eps=1e-3, fp64=False)
+    sample = np.random.default_rng(ns).choice(pos.shape[0], ns, replace=False)
+    got = plan.direct(sample)
+    plan.close()
+    ref = oracle.direct(pos[sample], pos, mass, soft_type=1, eps=1e-3)
+    pull = np.abs(ref).max()
+    assert np.abs(got - ref).max() < 4e4 * 2.0 ** -53 * pull, np.abs(got - ref).max() / pull

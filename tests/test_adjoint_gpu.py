@@ -157,3 +157,36 @@ def test_autograd_device_path_and_stale_plan(gpu_lib):
 def plan_adjoint_at(plan, pos, mass, w4):
     plan.update(pos, mass)
     return plan.adjoint(w4)
+
+
+@pytest.mark.parametrize("n,kw", [(3, dict(order=4, eps=0.05)), (70, dict(order=4, eps=0.05)),
+                                  (6000, dict(order=0)), (6000, dict(order=2)),
+                                  (6000, dict(order=4, merge_groups=5, rcb_cell=2048)),
+                                  (6000, dict(order=4, mac="tolerance", errtol=0.05))])
+def test_adjoint_along_a_direction(gpu_lib, n, kw):
+    """Every list kind (cells of orders 0, 2, 4 and bodies), lists shorter than the
+    waves that share them and longer: the gradient along a random direction against
+    the central difference of the FP64 forward.  With steps h and h/2 combined the
+    difference's own error is O(h^4); FP32 products leave a few 1e-7 of the summed
+    terms' magnitude, and each body's pair with itself, m w / eps^3 taken with both
+    signs, 2^-24 of that (eps keeps it below the bound)."""
+    from pgrav import batch, ics
+    pos, mass = ics.clustered(n, seed=41, nhalo=4)
+    rng = np.random.default_rng(10)
+    w4 = rng.normal(size=(n, 4))
+    kw = dict(dict(theta=0.6, eps=5e-3, soft="plummer", leaf_max=8), **kw)
+    plan = batch.Plan(pos, mass, **kw)
+    grad = plan.adjoint(w4)
+    dx, dm = rng.normal(size=(n, 3)), rng.normal(size=n) * 0.1
+
+    def loss(h):
+        plan.update(pos + h * dx, mass * (1 + h * dm))
+        plan.evaluate("f64")
+        return (plan.result("f64") * w4).sum()
+    h = 2e-5
+    d1 = (loss(h) - loss(-h)) / (2 * h)
+    d2 = (loss(h / 2) - loss(-h / 2)) / h
+    plan.close()
+    fd = (4 * d2 - d1) / 3
+    terms = np.concatenate([(grad[:, :3] * dx).ravel(), grad[:, 3] * mass * dm])
+    assert abs(terms.sum() - fd) < 1e-4 * np.linalg.norm(terms), (terms.sum(), fd, np.linalg.norm(terms))

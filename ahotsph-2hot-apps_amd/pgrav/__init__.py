@@ -119,12 +119,12 @@ class GravCuda:
         self._call("WalkTerminateSrcCUDA")
 
     def grav_mn(self, routine, first_body, m, f, source_n, sz, e, q):
-        p = ctypes.c_void_p(self.btab.ctypes.data + 4 * first_body * self.stride)
+        p = ctypes.c_void_p(ptr(self.btab).value + 4 * first_body * self.stride)
         self._call("grav_mn_CUDA", routine.encode(), p, None, m, self.stride, ptr(f), source_n,
                    sz, e, None, q)
 
     def pinteract(self, first_body, m, f, source_n, sz, q):
-        p = ctypes.c_void_p(self.btab.ctypes.data + 4 * first_body * self.stride)
+        p = ctypes.c_void_p(ptr(self.btab).value + 4 * first_body * self.stride)
         self._call("pinteractCUDA", p, None, m, self.stride, ptr(f), source_n, sz, q)
 
     def grav_mns(self, routine, base, m, seg, source_n, mmass, e, q):

@@ -5,6 +5,7 @@
 #include <stdint.h>
 
 #define NXCD 8      // MI355X accelerator complex dies (one L2 each)
+#define COUNTER_STRIDE 32  // ints between the persistent launch's work counters: a line each
 
 namespace pgrav {
 
@@ -37,7 +38,7 @@ struct BatchView {
     const uint8_t *img = nullptr;  // periodic = 2: image of each idx entry
     float4 *out32 = nullptr;
     double4 *out64 = nullptr;
-    int *counter = nullptr;
+    int *counter = nullptr;  // 2 + NXCD work counters, zero between launches
     double *far2 = nullptr;  // per group: square of its far distance (k_far); null: no expansions
     float4 *far_lo = nullptr;  // the far cells' pull: out32 and this remainder
     // the cell entries (and images) the expansions leave to the pair kernels, each list from
@@ -65,7 +66,6 @@ hipError_t launch_batch(const BatchView &v, int variant, int persistent_blocks, 
 // the far cells' pull into out32 and the groups' far distances into far2 (pgrav_far.hip)
 hipError_t launch_far(const BatchView &v, hipStream_t st);
 hipError_t launch_group64(const BatchView &v, int g, hipStream_t st);
-hipError_t launch_reset_counter(int *c, hipStream_t st);
 hipError_t launch_ewald_table(double L, double *t64, float *t32, hipStream_t st);
 // raw moment a (nln/cofm.c:660-720 order): its exponents e[a][q] and the index
 // of the moment with e[a][q] - 1 (when e[a][q] > 0)

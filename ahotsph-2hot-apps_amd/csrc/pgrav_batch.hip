@@ -517,7 +517,10 @@ void k_batch(BatchArgs A) {
 // cells -- run under one XCD's L2.  When its slice is drained it takes the
 // remaining groups of the other slices, so an XCD whose estimate was low does
 // not idle through the tail.  The last workgroup to leave resets the counters so
-// the launch can be replayed (e.g. from a graph).
+// the launch can be replayed (e.g. from a graph).  (With an atomic for a workgroup's
+// first group and for every drained slice, and all counters in one line, 512
+// workgroups queued 4,096 atomics on it: 65 us for 111 groups that take 33 now, 145 us
+// for 1,469 that take 122; looking before every atomic cost 25 % at 25,034 groups.)
 //
 // Every buffer also arrives as its own __restrict__ argument: the loop stores
 // a group's results and bumps the counters before it reads the next group's
@@ -548,38 +551,67 @@ void k_batch_persistent(
     extern __shared__ __align__(16) char smem[];
     __shared__ int w;
     const int x = blockIdx.x % NXCD;
-    // own slice first; once it is drained, the next group of the other XCDs' slices
-    // in turn (each counter only grows, so a drained slice stays drained)
-    int from = 0;
+    // the first groups of each slice are the workgroups' own, without a counter
+    const int given = gridDim.x / NXCD;
+    int item = A.xoff[x] + (int)blockIdx.x / NXCD;
+    bool own = item < A.xoff[x + 1];  // the own slice may have more groups
+    if (!own)
+        item = -1;
     for (;;) {
-        if (threadIdx.x == 0) {
-            int it = -1;
-            for (; from < NXCD; from++) {
-                const int xx = (x + from) % NXCD;
-                const int v = A.xoff[xx] + atomicAdd(&A.counter[2 + xx], 1);
-                if (v < A.xoff[xx + 1]) {
-                    it = v;
-                    break;
+        if (item < 0) {
+            // own slice first; once it is drained, the next group of the other XCDs' slices
+            // in turn (each counter only grows, so a drained slice stays drained: the other
+            // slices are looked at by a load, not by an atomic that every idle workgroup
+            // would queue for)
+            if (threadIdx.x < 64) {
+                const int lane = threadIdx.x, xl = (x + lane) % NXCD;
+                uint64_t left = own ? 1 : 0;  // slices to try, from x on
+                int it = -1;
+                for (;;) {
+                    while (left && it < 0) {
+                        const int k = __builtin_ctzll(left), xx = (x + k) % NXCD;
+                        left &= left - 1;
+                        int v = 0;
+                        if (lane == 0)
+                            v = A.xoff[xx] + given + atomicAdd(&A.counter[COUNTER_STRIDE * (2 + xx)], 1);
+                        v = __builtin_amdgcn_readfirstlane(v);
+                        if (v < A.xoff[xx + 1])
+                            it = v;
+                        else if (k == 0)
+                            own = false;
+                    }
+                    if (it >= 0)
+                        break;
+                    bool open = false;
+                    if (lane > 0 && lane < NXCD)
+                        open = given + __hip_atomic_load(&A.counter[COUNTER_STRIDE * (2 + xl)],
+                                                         __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) <
+                               A.xoff[xl + 1] - A.xoff[xl];
+                    left = __builtin_amdgcn_ballot_w64(open);
+                    if (!left)
+                        break;
                 }
+                if (lane == 0)
+                    w = it;
             }
-            w = it;
+            __syncthreads();
+            // the LDS value is the same in every lane: say so, so that the group's
+            // scalars (list offsets, record addresses) stay in SGPRs and the
+            // records keep coming through scalar loads
+            item = __builtin_amdgcn_readfirstlane(w);
+            __syncthreads();
+            if (item < 0)
+                break;
         }
-        __syncthreads();
-        // the LDS value is the same in every lane: say so, so that the group's
-        // scalars (list offsets, record addresses) stay in SGPRs and the
-        // records keep coming through scalar loads
-        const int item = __builtin_amdgcn_readfirstlane(w);
-        __syncthreads();
-        if (item < 0)
-            break;
         eval_group<T, REL, COMP, SOFT, PER, BU, TILE>(A, A.lpt[item],
                                                       (WaveShared<T, PER, TILE> *)smem);
+        item = -1;
     }
     if (threadIdx.x == 0) {
-        const int done = atomicAdd(&A.counter[1], 1);
+        const int done = atomicAdd(&A.counter[COUNTER_STRIDE], 1);
         if (done == (int)gridDim.x - 1) {
-            atomicExch(&A.counter[1], 0);
-            for (int k = 0; k < NXCD; k++) atomicExch(&A.counter[2 + k], 0);
+            atomicExch(&A.counter[COUNTER_STRIDE], 0);
+            for (int k = 0; k < NXCD; k++) atomicExch(&A.counter[COUNTER_STRIDE * (2 + k)], 0);
         }
     }
 }
@@ -589,11 +621,6 @@ template <int SOFT, int PER>
 __global__ __launch_bounds__(64) void k_group64(BatchArgs A, int g) {
     __shared__ WaveShared<double, PER, 64> shared[1];
     eval_group<double, false, false, SOFT, PER, 4>(A, g, shared);
-}
-
-__global__ void k_reset_counter(int *c) {
-    if (threadIdx.x < 2 + NXCD)
-        c[threadIdx.x] = 0;
 }
 
 // ---------------------------------------------------------------- FP64 direct sum
@@ -807,11 +834,6 @@ __global__ void k_ewald_table(double L, double *__restrict__ t64, float *__restr
 // ---------------------------------------------------------------- launchers
 hipError_t launch_ewald_table(double L, double *t64, float *t32, hipStream_t st) {
     hipLaunchKernelGGL(k_ewald_table, dim3((EWALD_NODES + 63) / 64), dim3(64), 0, st, L, t64, t32);
-    return hipGetLastError();
-}
-
-hipError_t launch_reset_counter(int *c, hipStream_t st) {
-    hipLaunchKernelGGL(k_reset_counter, dim3(1), dim3(64), 0, st, c);
     return hipGetLastError();
 }
 

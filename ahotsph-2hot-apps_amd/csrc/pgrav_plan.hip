@@ -461,8 +461,9 @@ void *pgrav_plan_create(const double *pos3, const double *mass, int64_t n, const
             if (p->periodic == 2)
                 P->v.near_img = P->dalloc<uint8_t>(cells);
         }
-        P->v.counter = P->dalloc<int>(64);
-        if (!check(hipMemset(P->v.counter, 0, 64), "hipMemset"))
+        const size_t cbytes = sizeof(int) * COUNTER_STRIDE * (2 + NXCD);
+        P->v.counter = P->dalloc<int>(cbytes);
+        if (!check(hipMemset(P->v.counter, 0, cbytes), "hipMemset"))
             throw std::runtime_error("memset");
         P->v.soft = p->soft_type;
         P->v.unroll = p->body_unroll ? p->body_unroll : 4;

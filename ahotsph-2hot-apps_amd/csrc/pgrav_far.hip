@@ -31,7 +31,6 @@ struct FarArgs {
     const int64_t *__restrict__ gslot_off;
     const uint32_t *__restrict__ gslot;
     const double4 *__restrict__ gcen;
-    const int *__restrict__ order;
     const int64_t *__restrict__ off;
     const uint32_t *__restrict__ idx;
     const uint8_t *__restrict__ img;
@@ -76,12 +75,27 @@ __device__ __forceinline__ void add_queued(const FarArgs &A, const FarShared &sh
     lx_add_cell<ORDER, SOFT, float>(rec, o.w, o.x, o.y, o.z, eps2, lam, acc);
 }
 
+// Workgroup b's group.  Workgroup b runs on XCD b mod NXCD: each XCD takes runs of
+// FAR_RUN groups, which are neighbours and share cells in its L2, dealt in turn.  (In the
+// pair kernel's slices, which are of equal cost in pairs and not in far cells, the XCDs
+// were busy for 78 % of the launch: clustered 16.8 M 27.8 ms with both kernels, 26.7 ms so,
+// and 1 M 1.86 and 1.76 ms; runs of 8 and of 128 within 1 % of it; a fixed grid that takes
+// its groups by counters from the slices, 27.0 and 1.81.)
+constexpr int FAR_RUN = 32;
+
+static __device__ __forceinline__ int group_of(int b, int ngroups) {
+    if (b >= ngroups / (NXCD * FAR_RUN) * (NXCD * FAR_RUN))
+        return b;
+    const int x = b % NXCD, i = b / NXCD;
+    return (i / FAR_RUN * NXCD + x) * FAR_RUN + i % FAR_RUN;
+}
+
 // (two waves per SIMD: the coefficients and a turned cell take 256 registers, and with
 // three the compiler's spills cost more than the third wave gives)
 template <bool SOFT, int PER>
 __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2))) void k_far(FarArgs A) {
     __shared__ FarShared sh;
-    const int g = A.order[blockIdx.x];
+    const int g = group_of(blockIdx.x, A.ngroups);
     const int lane = threadIdx.x;
     const int64_t G1 = A.ngroups + 1;
     int64_t ncell = 0;
@@ -233,7 +247,6 @@ hipError_t launch_far(const BatchView &v, hipStream_t st) {
     A.gslot_off = v.gslot_off;
     A.gslot = v.gslot;
     A.gcen = v.gcen;
-    A.order = v.order_np;
     A.off = v.off;
     A.idx = v.idx;
     A.img = v.img;

@@ -843,7 +843,9 @@ hipError_t launch_ewald_table(double L, double *t64, float *t32, hipStream_t st)
 // ends in a tail of long lists.  Four waves cost nothing where there are many groups;
 // eight and sixteen pay while the groups are few.  us per evaluation by 1, 2, 4, 8, 16
 // waves a group (order 4, theta 0.6 unless stated; in brackets: passes of two plans in
-// turn on two streams, where the tails overlap):
+// turn on two streams, where the tails overlap), every cell in pairs and before the
+// persistent launch's counters had a line each, which took sixteen waves to 33 us in the
+// first row and 122 in the second:
 //   111 groups (Plummer 4,099)            985   486   241   124    65
 //   1,469 (Plummer 65,536, order 2)      1049   525   280   178   143
 //   4,100 (lattice 64^3, images)         2054  1332  1176  1150  1139 [1713 .. 1051 1061 1073]

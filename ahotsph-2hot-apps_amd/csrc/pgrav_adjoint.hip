@@ -9,10 +9,11 @@
 // Every sum has one writer and a fixed order -- no atomics -- so two calls give
 // bit-identical gradients:
 //
-//  k_adjoint         one workgroup per sink group (lane = sink), the forward's tiling
-//                    and XCD-aware group order.  Per pair one derivative of the pull
-//                    along the sink's weight w gives the sink's gradient (closed
-//                    forms; dual numbers for the K1 bodies); the pair's source-side share (minus that, summed
+//  k_adjoint         one wave per sink group (lane = sink), the forward's tiling
+//                    and XCD-aware group order.  Per pair one forward-mode
+//                    derivative along the sink's weight w through the very same
+//                    cell_interact / mono_interact code gives the sink's
+//                    gradient; the pair's source-side share (minus that, summed
 //                    over the group's sinks, 8 entries at a time through LDS) is
 //                    written once per list entry: gpair (cells: dL/dX_c) and
 //                    gentry (bodies: dL/dx_j and dL/dm_j).
@@ -65,90 +66,6 @@ __device__ __forceinline__ D1 nrsq(D1 s) {
     return D1(f, -0.5f * f * f * f * s.d);
 }
 
-// J w - v a of one cell at the sink offset (x, y, z), (w, v) the sink's weights.  With
-// u = 1/(r^2 + eps^2), f = u^(1/2), P_k the record's harmonic polynomials, grad P_k =
-// k G_k, G_k' the derivative of G_k along w, q = x.w and t = u q,
-//   a = f sum_k u^k k G_k - beta x,  beta = f u sum_k u^k (2k+1) P_k,
-//   J w - v a = f sum_k u^k k (G_k' - ((2k+1) t + v) G_k) + (alpha + v beta) x - beta w,
-//   alpha = f u sum_k u^k (2k+1) ((2k+3) t P_k - k G_k.w),
-// the sums nested in u, so that no power of 1/r is formed that the forward kernel does not
-// form.  220 VALU instructions for order 4; the forward code run on (value, derivative)
-// pairs took 290.
-template <int ORDER>
-__device__ __forceinline__ void cell_pull_gradient(const float *__restrict__ M, float m, float x,
-                                                   float y, float z, float eps2, float4 w, float &px,
-                                                   float &py, float &pz) {
-    const float x2 = x * x, y2 = y * y, z2 = z * z;
-    const float f = -nrsq(x2 + y2 + z2 + eps2), u = f * f, fu = f * u;
-    const float t = u * (x * w.x + y * w.y + z * w.z), v = w.w;
-    float beta = m, alpha = 3.0f * t * m;
-    float ax = 0.f, ay = 0.f, az = 0.f;
-    if constexpr (ORDER >= 2) {
-        float bs = 0.f, as = 0.f, hx = 0.f, hy = 0.f, hz = 0.f;  // orders 3 and 4
-        if constexpr (ORDER >= 4) {
-            const float xy = x * y, xz = x * z, yz = y * z;
-            const float A = x2 - z2, B = y2 - z2;
-            const float zw = z * w.z;
-            const float dA = 2.0f * (x * w.x - zw), dB = 2.0f * (y * w.y - zw);
-            const float dxy = x * w.y + y * w.x, dxz = x * w.z + z * w.x, dyz = y * w.z + z * w.y;
-            {
-                const float z3 = 3.0f * z2;
-                const float U1 = x * (x2 - z3), U2 = y * (y2 - z3), U3 = y * A,
-                            U4 = z * (3.0f * x2 - z2), U5 = x * B, U6 = xy * z, U7 = z * (3.0f * y2 - z2);
-                const float A3 = 3.0f * A, B3 = 3.0f * B, xz6 = 6.0f * xz, yz6 = 6.0f * yz;
-                const float V1 = A3 * w.x - xz6 * w.z, V2 = B3 * w.y - yz6 * w.z, V3 = A * w.y + y * dA,
-                            V4 = xz6 * w.x + A3 * w.z, V5 = B * w.x + x * dB, V6 = z * dxy + xy * w.z,
-                            V7 = yz6 * w.y + B3 * w.z;
-                const float *h = M + 25;
-                const float g0 = h[0] * U1 + h[1] * U2 + h[2] * U3 + h[3] * U4 + h[4] * U5 + h[5] * U6 + h[6] * U7;
-                const float g1 = h[7] * U1 + h[8] * U2 + h[9] * U3 + h[10] * U4 + h[11] * U5 + h[12] * U6 + h[13] * U7;
-                const float g2 = h[14] * U1 + h[15] * U2 + h[16] * U3 + h[17] * U4 + h[18] * U5 + h[19] * U6 + h[20] * U7;
-                const float d0 = h[0] * V1 + h[1] * V2 + h[2] * V3 + h[3] * V4 + h[4] * V5 + h[5] * V6 + h[6] * V7;
-                const float d1 = h[7] * V1 + h[8] * V2 + h[9] * V3 + h[10] * V4 + h[11] * V5 + h[12] * V6 + h[13] * V7;
-                const float d2 = h[14] * V1 + h[15] * V2 + h[16] * V3 + h[17] * V4 + h[18] * V5 + h[19] * V6 + h[20] * V7;
-                const float p = g0 * x + g1 * y + g2 * z, gw = g0 * w.x + g1 * w.y + g2 * w.z;
-                const float e = 9.0f * t + v, u4 = 4.0f * u;
-                bs = u * (9.0f * p);
-                as = u * (99.0f * (t * p) - 36.0f * gw);
-                hx = u4 * (d0 - e * g0);
-                hy = u4 * (d1 - e * g1);
-                hz = u4 * (d2 - e * g2);
-            }
-            const float *o = M + 10;
-            const float g0 = o[0] * A + o[1] * B + o[2] * xy + o[3] * xz + o[4] * yz;
-            const float g1 = o[5] * A + o[6] * B + o[7] * xy + o[8] * xz + o[9] * yz;
-            const float g2 = o[10] * A + o[11] * B + o[12] * xy + o[13] * xz + o[14] * yz;
-            const float d0 = o[0] * dA + o[1] * dB + o[2] * dxy + o[3] * dxz + o[4] * dyz;
-            const float d1 = o[5] * dA + o[6] * dB + o[7] * dxy + o[8] * dxz + o[9] * dyz;
-            const float d2 = o[10] * dA + o[11] * dB + o[12] * dxy + o[13] * dxz + o[14] * dyz;
-            const float p = g0 * x + g1 * y + g2 * z, gw = g0 * w.x + g1 * w.y + g2 * w.z;
-            const float e = 7.0f * t + v;
-            bs = u * (7.0f * p + bs);
-            as = u * (63.0f * (t * p) + (as - 21.0f * gw));
-            hx = u * (3.0f * (d0 - e * g0) + hx);
-            hy = u * (3.0f * (d1 - e * g1) + hy);
-            hz = u * (3.0f * (d2 - e * g2) + hz);
-        }
-        const float gx = M[4] * x + M[5] * y + M[6] * z, gy = M[5] * x + M[7] * y + M[8] * z,
-                    gz = M[6] * x + M[8] * y + M[9] * z;
-        const float dx = M[4] * w.x + M[5] * w.y + M[6] * w.z, dy = M[5] * w.x + M[7] * w.y + M[8] * w.z,
-                    dz = M[6] * w.x + M[8] * w.y + M[9] * w.z;
-        const float p = gx * x + gy * y + gz * z, gw = gx * w.x + gy * w.y + gz * w.z;
-        const float e = 5.0f * t + v, uu = u * u, fuu = fu * u;
-        beta += uu * (5.0f * p + bs);
-        alpha += uu * (35.0f * (t * p) + (as - 10.0f * gw));
-        ax = fuu * (2.0f * (dx - e * gx) + hx);
-        ay = fuu * (2.0f * (dy - e * gy) + hy);
-        az = fuu * (2.0f * (dz - e * gz) + hz);
-    }
-    beta *= fu;
-    const float c = fu * alpha + v * beta;
-    px = ax + c * x - beta * w.x;
-    py = ay + c * y - beta * w.y;
-    pz = az + c * z - beta * w.z;
-}
-
-#define ADJ_WAVES 3  // waves that share a group's lists (9 KB of LDS each)
 #define ADJ_CELL 52  // per work item / node: 46 dL/dP, 3 dL/dX (pair part), pad
 #define L_BODY_KIND 3  // list kinds 0..2 are cells (orders 4, 2, 0), 3 bodies
 
@@ -218,8 +135,8 @@ __device__ __forceinline__ int64_t sink_slot(const BatchView &V, int64_t ref, in
 // and lane 8 s writes entry s: out[base + s], s < n.
 __device__ __forceinline__ void flush_entries(float4 (*red)[64], int n, float4 *__restrict__ out,
                                               int64_t base) {
-    wave_sync();
-    const int lane = threadIdx.x & 63, s = lane >> 3, p = lane & 7;
+    __syncthreads();
+    const int lane = threadIdx.x, s = lane >> 3, p = lane & 7;
     float ax = 0.f, ay = 0.f, az = 0.f, aw = 0.f;
 #pragma unroll
     for (int i = 0; i < 8; i++) {
@@ -235,28 +152,20 @@ __device__ __forceinline__ void flush_entries(float4 (*red)[64], int n, float4 *
     aw = dpp_add<0x141, 0xf>(dpp_add<0x4e, 0xf>(dpp_add<0xb1, 0xf>(aw)));
     if (p == 0 && s < n)
         out[base + s] = make_float4(ax, ay, az, aw);
-    wave_sync();
+    __syncthreads();
 }
 
 // Every buffer arrives as its own __restrict__ argument: the kernel stores
 // entry results between its reads of the lists and records, and only pointers
 // known to be distinct let the compiler read those through scalar loads.
 //
-// Three waves share a group's lists: the first takes the bodies, the others half of
-// every cell list each (~35 VALU an entry against ~225), and the sinks' sums meet in
-// LDS.  The bodies stay with one wave, in list order, because their sum is the ill-
-// conditioned one: a body's pair with itself, m w / eps^3, cancels only against its
-// source side later, so another order of the additions after it is another rounding of
-// a large number (7e-5 of the gradient at 262,144 bodies with eps 1e-4).  us per adjoint
-// in all with one wave and with 2, 3, 4, clustered bodies: 8,192 548, 420 420 420;
-// 262,144 4168, 3338 3255 3299; its bisection groups 3680, 2896 3027 3107; 1 M 17.2 ms,
-// 17.1 16.4 15.5.
-struct AdjointWave {
-    float4 tile[64];
-    float4 red[8][64];
-};
+// A sink's sum is FP32 and takes its cells, then its bodies, in list order.  The order
+// is part of the result: a body's pair with itself (m w / eps^3; K1: 11 m w / eps^3) is
+// cancelled only by its source side, in k_adjoint_bodies, and every addition after it
+// rounds at its size (eps 1e-4, 2,000 to 40,000 bodies: another order moves the
+// gradient by 1e-4 to 6e-1).  So one wave takes all of a group's lists.
 template <int SOFT>
-__global__ __launch_bounds__(64 * ADJ_WAVES) void k_adjoint(
+__global__ __launch_bounds__(64) void k_adjoint(
     BatchView V, AdjointView A, const int *__restrict__ order, const int *__restrict__ gcount,
     const double4 *__restrict__ gcen, const int64_t *__restrict__ gfirst,
     const int64_t *__restrict__ gslot_off, const uint32_t *__restrict__ gslot,
@@ -264,15 +173,13 @@ __global__ __launch_bounds__(64 * ADJ_WAVES) void k_adjoint(
     const float *__restrict__ mom, const double4 *__restrict__ bpos,
     const double4 *__restrict__ cpos, const float4 *__restrict__ wv, float4 *__restrict__ gpair,
     float4 *__restrict__ gentry, float4 *__restrict__ gsink) {
-    __shared__ AdjointWave shared[ADJ_WAVES];
-    const int w64 = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
-    float4 *lds = shared[w64].tile;
-    float4(*red)[64] = shared[w64].red;
+    __shared__ float4 lds[64];
+    __shared__ float4 red[8][64];
     // XCD-aware order: consecutive workgroups land on different XCDs, so the
     // forward's per-XCD slices of Morton-neighbouring groups keep their cells in
     // one XCD's L2 here too
     const int g = order ? order[blockIdx.x] : (int)blockIdx.x;
-    const int lane = threadIdx.x & 63;
+    const int lane = threadIdx.x;
     const int cnt = gcount[g];
     const double4 gc = gcen[g];
     const bool live = lane < cnt;
@@ -289,40 +196,34 @@ __global__ __launch_bounds__(64 * ADJ_WAVES) void k_adjoint(
 
     for (int kind = 0; kind < 4; kind++) {
         const int64_t *offk = off + (int64_t)kind * (V.ngroups + 1);
-        const int64_t l0 = offk[g], l1 = offk[g + 1];
-        int64_t o0 = l0, o1 = w64 ? l0 : l1;  // the bodies
-        if (kind < L_BODY_KIND) {
-            const int64_t share = (l1 - l0 + ADJ_WAVES - 2) / (ADJ_WAVES - 1);
-            o0 = w64 ? min(l1, l0 + (w64 - 1) * share) : l1;
-            o1 = min(l1, o0 + share);
-        }
+        const int64_t o0 = offk[g], o1 = offk[g + 1];
         for (int64_t t0 = o0; t0 < o1; t0 += 64) {
             const int nt = (int)min((int64_t)64, o1 - t0);
-            // (past the end: massless bodies, so that the blocks of 8 need no branch)
-            float4 src = make_float4(0.f, 0.f, 0.f, 0.f);
             if (lane < nt) {
                 const uint32_t e = idx[t0 + lane];
                 const double4 s = kind == 3 ? bpos[e] : cpos[e];
-                src = make_float4((float)(s.x - gc.x), (float)(s.y - gc.y), (float)(s.z - gc.z),
-                                  (float)s.w);
+                lds[lane] = make_float4((float)(s.x - gc.x), (float)(s.y - gc.y),
+                                        (float)(s.z - gc.z), (float)s.w);
             }
-            lds[lane] = src;
-            wave_sync();
+            __syncthreads();
             if (kind < L_BODY_KIND) {
                 for (int k = 0; k < nt; k++) {
                     const float4 r = lds[k];
-                    const float X = sx - r.x, Y = sy - r.y, Z = sz - r.z;
+                    // the sink offset, differentiated along this sink's weight w
+                    const D1 dx(sx - r.x, w.x), dy(sy - r.y, w.y), dz(sz - r.z, w.z);
+                    Acc4T<D1> a = {D1(0.f), D1(0.f), D1(0.f), D1(0.f)};
                     const uint32_t e = idx[t0 + k];
+                    if (kind == 0)
+                        cell_interact<4, false, 1, D1, float>(mom + (size_t)e * PREC4, D1(r.w), dx, dy, dz, D1(eps2c), a);
+                    else if (kind == 1)
+                        cell_interact<2, false, 1, D1, float>(mom + (size_t)e * PREC4, D1(r.w), dx, dy, dz, D1(eps2c), a);
+                    else
+                        mono_interact<D1>(D1(r.w), dx, dy, dz, D1(eps2c), a);
                     // d(w.a + v phi)/d(sink position) = J w - v a; the cell's centre
                     // takes minus that, summed over the group's sinks
-                    float px, py, pz;
-                    const float *M = mom + (size_t)e * PREC4;
-                    if (kind == 0)
-                        cell_pull_gradient<4>(M, r.w, X, Y, Z, eps2c, w, px, py, pz);
-                    else if (kind == 1)
-                        cell_pull_gradient<2>(M, r.w, X, Y, Z, eps2c, w, px, py, pz);
-                    else
-                        cell_pull_gradient<0>(M, r.w, X, Y, Z, eps2c, w, px, py, pz);
+                    const float px = a.x.d - w.w * a.x.v;
+                    const float py = a.y.d - w.w * a.y.v;
+                    const float pz = a.z.d - w.w * a.z.v;
                     gx += px;
                     gy += py;
                     gz += pz;
@@ -337,60 +238,47 @@ __global__ __launch_bounds__(64 * ADJ_WAVES) void k_adjoint(
                     const int m = min(8, nt - k0);
 #pragma unroll
                     for (int i = 0; i < 8; i++) {
-                        const float4 r = lds[k0 + i];  // k0 + i < 64
-                        const float X = sx - r.x, Y = sy - r.y, Z = sz - r.z;
-                        float px, py, pz, pm;
-                        if (SOFT == SOFT_K1) {
-                            const D1 dx(X, w.x), dy(Y, w.y), dz(Z, w.z);
-                            Acc4T<D1> a = {D1(0.f), D1(0.f), D1(0.f), D1(0.f)};
-                            // unit mass: the pair is linear in the source mass
-                            k1_interact<D1>(D1(1.f), dx, dy, dz, D1(eps_inv), D1(eps2), a);
-                            px = r.w * (a.x.d - w.w * a.x.v);
-                            py = r.w * (a.y.d - w.w * a.y.v);
-                            pz = r.w * (a.z.d - w.w * a.z.v);
-                            pm = w.x * a.x.v + w.y * a.y.v + w.z * a.z.v + w.w * a.w.v;
-                        } else {
-                            // Plummer (or none): with f = 1/sqrt(r^2 + eps^2), a = -m f^3 x and
-                            // phi = -m f, so J w - v a = m f^3 ((3 f^2 x.w + v) x - w) and
-                            // d(w.a + v phi)/dm = -(f^3 x.w + v f); the unsoftened self pair is 0
-                            const float r2 = fmaf(X, X, fmaf(Y, Y, fmaf(Z, Z, eps2c)));
-                            const bool self = SOFT == SOFT_NONE && r2 == 0.f;
-                            const float f = self ? 0.f : __builtin_amdgcn_rsqf(r2);
-                            const float f2 = f * f, f3 = f2 * f;
-                            const float xw = w.x * X + w.y * Y + w.z * Z;
-                            const float t = 3.0f * f2 * xw + w.w;
-                            const float mf3 = r.w * f3;
-                            px = mf3 * (t * X - w.x);
-                            py = mf3 * (t * Y - w.y);
-                            pz = mf3 * (t * Z - w.z);
-                            pm = -(f3 * xw + w.w * f);
+                        const float4 r = lds[k0 + i];  // k0 + i < 64: inside the tile buffer
+                        if (i < m) {
+                            const float X = sx - r.x, Y = sy - r.y, Z = sz - r.z;
+                            float px, py, pz, pm;
+                            if (SOFT == SOFT_K1) {
+                                const D1 dx(X, w.x), dy(Y, w.y), dz(Z, w.z);
+                                Acc4T<D1> a = {D1(0.f), D1(0.f), D1(0.f), D1(0.f)};
+                                // unit mass: the pair is linear in the source mass
+                                k1_interact<D1>(D1(1.f), dx, dy, dz, D1(eps_inv), D1(eps2), a);
+                                px = r.w * (a.x.d - w.w * a.x.v);
+                                py = r.w * (a.y.d - w.w * a.y.v);
+                                pz = r.w * (a.z.d - w.w * a.z.v);
+                                pm = w.x * a.x.v + w.y * a.y.v + w.z * a.z.v + w.w * a.w.v;
+                            } else {
+                                // Plummer (or none): with f = 1/sqrt(r^2 + eps^2), a = -m f^3 x and
+                                // phi = -m f, so J w - v a = m f^3 ((3 f^2 x.w + v) x - w) and
+                                // d(w.a + v phi)/dm = -(f^3 x.w + v f); the unsoftened self pair is 0
+                                const float r2 = fmaf(X, X, fmaf(Y, Y, fmaf(Z, Z, eps2c)));
+                                const bool self = SOFT == SOFT_NONE && r2 == 0.f;
+                                const float f = self ? 0.f : __builtin_amdgcn_rsqf(r2);
+                                const float f2 = f * f, f3 = f2 * f;
+                                const float xw = w.x * X + w.y * Y + w.z * Z;
+                                const float t = 3.0f * f2 * xw + w.w;
+                                const float mf3 = r.w * f3;
+                                px = mf3 * (t * X - w.x);
+                                py = mf3 * (t * Y - w.y);
+                                pz = mf3 * (t * Z - w.z);
+                                pm = -(f3 * xw + w.w * f);
+                            }
+                            gx += px;
+                            gy += py;
+                            gz += pz;
+                            red[i][lane] = make_float4(-px, -py, -pz, pm);
                         }
-                        gx += px;
-                        gy += py;
-                        gz += pz;
-                        red[i][lane] = make_float4(-px, -py, -pz, pm);
                     }
                     flush_entries(red, m, gentry, t0 + k0 - ncell);
                 }
             }
-            wave_sync();
+            __syncthreads();
         }
     }
-    if (w64)
-        lds[lane] = make_float4(gx, gy, gz, 0.f);
-    __syncthreads();
-    if (w64)
-        return;
-    float4 c = shared[1].tile[lane];
-    for (int k = 2; k < ADJ_WAVES; k++) {
-        const float4 v = shared[k].tile[lane];
-        c.x += v.x;
-        c.y += v.y;
-        c.z += v.z;
-    }
-    gx += c.x;
-    gy += c.y;
-    gz += c.z;
     if (live)
         gsink[me] = make_float4(gx, gy, gz, 0.f);
 }
@@ -674,8 +562,8 @@ hipError_t launch_adjoint(const BatchView &v, const AdjointView &A, hipStream_t 
     if (v.ngroups <= 0)
         return hipSuccess;
 #define ADJ(S)                                                                                     \
-    hipLaunchKernelGGL(k_adjoint<S>, dim3(v.ngroups), dim3(64 * ADJ_WAVES), 0, st, v, A, v.order_np,  \
-                       v.gcount, v.gcen, v.gfirst, v.gslot_off, v.gslot, v.off, v.idx, v.mom32, v.bpos,     \
+    hipLaunchKernelGGL(k_adjoint<S>, dim3(v.ngroups), dim3(64), 0, st, v, A, v.order_np, v.gcount, \
+                       v.gcen, v.gfirst, v.gslot_off, v.gslot, v.off, v.idx, v.mom32, v.bpos,     \
                        v.cpos, A.wv, A.gpair, A.gentry, A.gsink);                                 \
     if (A.ntcells > 0 && v.gslot)                                                                  \
         hipLaunchKernelGGL((k_adjoint_cells<S, true>), dim3(A.ntcells), dim3(64), 0, st, v, A);    \

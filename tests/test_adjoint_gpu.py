@@ -190,3 +190,111 @@ def test_adjoint_along_a_direction(gpu_lib, n, kw):
     fd = (4 * d2 - d1) / 3
     terms = np.concatenate([(grad[:, :3] * dx).ravel(), grad[:, 3] * mass * dm])
     assert abs(terms.sum() - fd) < 1e-4 * np.linalg.norm(terms), (terms.sum(), fd, np.linalg.norm(terms))
+
+
+def test_unsoftened_sink_beside_the_group_centre(gpu_lib):
+    """Three bodies in a row, one group: the middle one misses the centre by a rounding
+    error, so that anything evaluated at the centre itself (a block's unused entries)
+    overflows.  Against the FP64 direct gradient; one pair's FP32 products a few 2^-24."""
+    from pgrav import batch
+    pos, mass = np.array([[.1, .1, .1], [.4, .1, .1], [.7, .1, .1]]), np.array([.2, .3, .5])
+    kw = dict(soft="none", eps=0.0, order=4)
+    c = batch.HostPlan(pos, mass, **kw).group(0)[2]
+    assert 0 < abs(c[0] - pos[1, 0]) < 1e-15
+    w4 = np.random.default_rng(4).normal(size=(3, 4))
+    plan = batch.Plan(pos, mass, **kw)
+    grad = plan.adjoint(w4)
+    plan.close()
+    ref = oracle.direct_grad(pos, mass, w4, soft_type=0, eps=0.0)
+    assert np.abs(grad - ref).max() < 64 * 2.0 ** -24 * np.abs(ref).max(), (grad, ref)
+
+
+def _pair(r2, eps):
+    """(phi, e, e') of a unit mass at distance sqrt(r2): a = e d, e' = 2 de/d(r2); Dehnen's
+    K1 inside eps (0: none).  The pair at zero distance of an unsoftened body is 0."""
+    f = np.where(r2 > 0, np.maximum(r2, 1e-300) ** -0.5, 0.0)
+    phi, e, de = -f, -f ** 3, 3 * f ** 5
+    if eps:
+        u, near = r2 / eps ** 2 - 1, r2 <= eps ** 2
+        phi = np.where(near, (((45 / 32 * u - 3 / 8) * u + 0.5) * u - 1) / eps, phi)
+        e = np.where(near, ((-135 / 16 * u + 1.5) * u - 1) / eps ** 3, e)
+        de = np.where(near, (-135 / 4 * u + 3) / eps ** 5, de)
+    return phi, e, de
+
+
+def _pair_gradients(d, m, w, eps):
+    """J w - v a of pairs at d = sink - source; w the sinks' weights (w, v)."""
+    _, e, de = _pair((d * d).sum(-1), eps)
+    q = (d * w[..., :3]).sum(-1)
+    return (m * e)[..., None] * (w[..., :3] - w[..., 3:] * d) + (m * de * q)[..., None] * d
+
+
+@pytest.mark.parametrize("soft,eps", [("k1", 5e-3), ("none", 0.0)])
+def test_k1_and_unsoftened_gradients(gpu_lib, soft, eps):
+    """As the Plummer-softened test, against the FP64 direct sum: the tree's own error at
+    theta 0.4, order 4 (K1: eps such that a body's pair with itself, 11 m w / eps^3, leaves
+    less than that behind: 2^-24 x 2e4 beside gradients of 1e2)."""
+    from pgrav import batch, ics
+    n = 4096
+    pos, mass = ics.clustered(n, seed=32, nhalo=8)
+    w4 = np.random.default_rng(6).normal(size=(n, 4))
+    plan = batch.Plan(pos, mass, theta=0.4, order=4, eps=eps, soft=soft)
+    grad = plan.adjoint(w4)
+    plan.close()
+    ref = np.zeros((n, 4))
+    for i in range(0, n, 256):
+        d = pos[i:i + 256, None] - pos[None]
+        p = _pair_gradients(d, mass[None], w4[i:i + 256, None], eps)
+        ref[i:i + 256, :3] += p.sum(1)
+        ref[:, :3] -= p.sum(0)
+        phi, e, _ = _pair((d * d).sum(-1), eps)
+        ref[:, 3] += (e * (d * w4[i:i + 256, None, :3]).sum(-1) + phi * w4[i:i + 256, None, 3]).sum(0)
+    dx = np.linalg.norm(grad[:, :3] - ref[:, :3], axis=1) / np.linalg.norm(ref[:, :3], axis=1)
+    dm = np.abs(grad[:, 3] - ref[:, 3]) / np.abs(ref[:, 3])
+    assert np.median(dx) < 1e-3 and np.median(dm) < 1e-3, (np.median(dx), np.median(dm))
+
+
+def test_adjoint_adds_in_its_stated_order(gpu_lib):
+    """A sink's FP32 sum takes its cells, then its bodies, each in list order.  Softened
+    closely, a body's pair with itself (11 m w / eps^3, K1) is larger than all others by
+    1e7 until its source side cancels it, so that what is left depends on that order: the
+    same sum in numpy, for one weighted sink at a time, whose gradient is then its own sum
+    less that pair.  Every term after the own pair rounds on the pair's grid, a fifth of
+    the terms; no body has another inside eps, so that the pair terms' 1e-7 hardly ever
+    moves such a rounding, while another order moves three in ten of the sums.  (Masses and
+    eps are powers of two and weights short, so that the own pair is exact, fused or not.)"""
+    from pgrav import batch
+    eps, f32, n = 2.0 ** -9, np.float32, 729
+    rng = np.random.default_rng(3)
+    pos = (np.stack(np.meshgrid(*[np.arange(9)] * 3, indexing="ij"), -1).reshape(-1, 3) +
+           rng.uniform(0.3, 0.7, (n, 3))) / 9
+    mass = np.full(n, 2.0 ** -10)
+    kw = dict(theta=0.7, order=0, eps=eps, soft="k1", leaf_max=8, group_max=32)
+    host = batch.HostPlan(pos, mass, **kw)
+    perm, spos = host.sorted()
+    w4 = np.round(rng.normal(size=(n, 4)) * 256) / 256
+    plan = batch.Plan(pos, mass, **kw)
+    same = []
+    for g in range(host.stats()["ngroups"]):
+        first, cnt, c = host.group(g)
+        cells, bodies = [host.cell(k) for k in host.list(g, "mono")], host.list(g, "body")
+        assert len(cells) and len(host.list(g, "hexa")) == 0
+        for i in {first, first + cnt // 2}:
+            w = w4[i]
+
+            def terms(p, m, e):
+                d = ((spos[i] - c[:3]).astype(f32) - (p - c[:3]).astype(f32)).astype(np.float64)
+                return _pair_gradients(d, m.astype(f32).astype(np.float64), w, e).astype(f32)
+            pc = terms(np.array([k["cofm"] for k in cells]), np.array([k["raw"][0] for k in cells]), 0)
+            pb = terms(spos[bodies], mass[perm[bodies]], float(f32(eps)))
+            own = pb[np.flatnonzero(bodies == i)[0]]
+            want = np.zeros(3, f32)
+            for t in np.concatenate([pc, pb]):
+                want = want + t
+            want = want - own
+            one = np.zeros((n, 4))
+            one[perm[i]] = w
+            got = plan.adjoint(one)[perm[i], :3]
+            same += list(np.abs(got - want) < 0.5 * np.spacing(np.abs(own)))
+    plan.close()
+    assert np.mean(same) > 0.93, np.mean(same)

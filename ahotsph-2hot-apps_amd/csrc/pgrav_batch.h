@@ -40,7 +40,7 @@ struct BatchView {
     double4 *out64 = nullptr;
     int *counter = nullptr;  // 2 + NXCD work counters, zero between launches
     double *far2 = nullptr;  // per group: square of its far distance (k_far); null: no expansions
-    float4 *far_lo = nullptr;  // the far cells' pull: out32 and this remainder
+    float4 *far_pull = nullptr;  // [n][2], by slot: the far cells' pull, rounded and the remainder
     // the cell entries (and images) the expansions leave to the pair kernels, each list from
     // its own start in idx, and their number [3][ngroups]
     uint32_t *near = nullptr;
@@ -63,7 +63,7 @@ struct BatchView {
 };
 
 hipError_t launch_batch(const BatchView &v, int variant, int persistent_blocks, hipStream_t st);
-// the far cells' pull into out32 and the groups' far distances into far2 (pgrav_far.hip)
+// the far cells' pull into far_pull and the groups' far distances into far2 (pgrav_far.hip)
 hipError_t launch_far(const BatchView &v, hipStream_t st);
 hipError_t launch_group64(const BatchView &v, int g, hipStream_t st);
 hipError_t launch_ewald_table(double L, double *t64, float *t32, hipStream_t st);

@@ -64,7 +64,7 @@ struct BatchArgs {
     int unroll;          // order-0 / body loop unroll of the rel32c kernels: 2, 4 or 8
     int tile;            // list entries staged in LDS per round (rel32c, not periodic 1): 32, 64, 128
     const double *far2;  // per group: square of its far distance (null: no expansions)
-    const float4 *far_lo;  // the far cells' pull: out and this remainder
+    const float4 *far_pull;  // the far cells' pull at each slot: rounded and the remainder
     // what the expansion leaves of the cell lists (periodic 1: the kernel decides itself)
     const uint32_t *near;
     const uint8_t *near_img;
@@ -274,8 +274,7 @@ __device__ __forceinline__ void eval_group(const BatchArgs &A, int g,
         if (A.far2)
             far2 = A.far2[g];
         if (far2 < (double)INFINITY && w == 0) {  // the far cells' pull at this sink (k_far)
-            const V4<T> f = ((const V4<T> *)A.out)[slot];
-            const float4 lo = A.far_lo[slot];
+            const float4 f = A.far_pull[2 * slot], lo = A.far_pull[2 * slot + 1];
             s = Acc4T<T>{f.x, f.y, f.z, f.w};
             if (COMP)
                 c = Acc4T<T>{lo.x, lo.y, lo.z, lo.w};
@@ -949,13 +948,13 @@ hipError_t launch_batch(const BatchView &v, int variant, int persistent_blocks, 
     A.tile = v.tile;
     A.ewratio = v.ewratio;
     A.far2 = nullptr;
-    A.far_lo = nullptr;
+    A.far_pull = nullptr;
     A.near = nullptr;
     A.near_img = nullptr;
     A.near_n = nullptr;
     if ((variant == VAR_REL32C || variant == VAR_REL32) && v.far2) {
         A.far2 = v.far2;
-        A.far_lo = v.far_lo;
+        A.far_pull = v.far_pull;
         A.near = v.near;
         A.near_img = v.near_img;
         A.near_n = v.near_n;
@@ -1010,7 +1009,7 @@ hipError_t launch_group64(const BatchView &v, int g, hipStream_t st) {
     A.tile = v.tile;
     A.ewratio = v.ewratio;
     A.far2 = nullptr;
-    A.far_lo = nullptr;
+    A.far_pull = nullptr;
     A.near = nullptr;
     A.near_img = nullptr;
     A.near_n = nullptr;

@@ -6,7 +6,9 @@
 // every lane, each lane takes one cell: it gathers the cell's record and adds the
 // cell's expansion to its own 81 (softened: 101) coefficients in registers.  The lanes'
 // coefficients meet through LDS in a fixed order, and their sum is evaluated at the
-// group's sinks into the result array, from where the pair kernel takes it up.
+// group's sinks into a buffer of its own, from where the pair kernel takes it up: the
+// result array only ever holds whole results, so that a reader of the last evaluation's
+// on another stream sees the same values while the next one of the same bodies runs.
 //
 // Bound by VALU at two waves per SIMD: 1,500 instructions per 64 order-4 cells (1,050
 // order 2, 345 order 0) against 110 (45, 16) x 64 in pairs, ~110 per 64 entries scanned
@@ -40,7 +42,7 @@ struct FarArgs {
     uint32_t *__restrict__ near;  // the entries left to the pair kernel, at their list's start
     uint8_t *__restrict__ near_img;
     int *__restrict__ near_n;  // [3][ngroups]
-    float4 *__restrict__ out, *__restrict__ lo;
+    float4 *__restrict__ pull;  // [n][2]
 };
 
 constexpr int ROWS = 16;  // coefficients summed over the lanes per LDS round
@@ -225,9 +227,9 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2))) void k_
         const double v[4] = {gx + r[0], gy + r[1], gz + r[2],
                              r[3] - (a[0] + gx * sx + gy * sy + gz * sz)};
         const float4 hi = make_float4((float)v[0], (float)v[1], (float)v[2], (float)v[3]);
-        A.out[slot] = hi;
-        A.lo[slot] = make_float4((float)(v[0] - hi.x), (float)(v[1] - hi.y), (float)(v[2] - hi.z),
-                                 (float)(v[3] - hi.w));
+        A.pull[2 * slot] = hi;
+        A.pull[2 * slot + 1] = make_float4((float)(v[0] - hi.x), (float)(v[1] - hi.y),
+                                           (float)(v[2] - hi.z), (float)(v[3] - hi.w));
     }
 }
 
@@ -257,8 +259,7 @@ hipError_t launch_far(const BatchView &v, hipStream_t st) {
     A.ibox = 1.0 / v.box;
     A.ewratio = v.ewratio;
     A.far2 = v.far2;
-    A.out = v.out32;
-    A.lo = v.far_lo;
+    A.pull = v.far_pull;
     A.near = v.near;
     A.near_img = v.near_img;
     A.near_n = v.near_n;

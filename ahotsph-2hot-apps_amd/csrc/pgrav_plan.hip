@@ -455,7 +455,7 @@ void *pgrav_plan_create(const double *pos3, const double *mass, int64_t n, const
             int64_t cells = 0;
             for (int k = 0; k < L_BODY; k++) cells += L.off[k].back();
             P->v.far2 = P->dalloc<double>(sizeof(double) * G);
-            P->v.far_lo = P->dalloc<float4>(sizeof(float4) * (size_t)n);
+            P->v.far_pull = P->dalloc<float4>(2 * sizeof(float4) * (size_t)n);
             P->v.near_n = P->dalloc<int>(sizeof(int) * 3 * G);
             P->v.near = P->dalloc<uint32_t>(sizeof(uint32_t) * cells);
             if (p->periodic == 2)

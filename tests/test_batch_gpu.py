@@ -350,6 +350,29 @@ def test_far_cells_match_the_pairs(gpu_lib, kw):
     plan.close()
 
 
+def test_results_stay_whole_under_the_next_evaluation(gpu_lib):
+    """A result read on one stream while the same bodies are evaluated again on another:
+    the result array holds whole sums only, so every read gives the first one's values."""
+    import torch
+    from pgrav import batch, ics
+    pos, mass = ics.clustered(60000, seed=21, nhalo=24)
+    plan = batch.Plan(pos, mass, theta=0.6, order=4, eps=1e-3, group_max=8, leaf_max=16)
+    assert _far_pays(plan.stats(), False)
+    s1, s2 = torch.cuda.Stream(), torch.cuda.Stream()
+    acc = torch.empty((8, 60000, 4), dtype=torch.float32, device="cuda")
+    torch.cuda.synchronize()
+    plan.evaluate("rel32c", stream=s1.cuda_stream)
+    want = plan.result("rel32c")
+    for k in range(8):
+        plan.result_device("rel32c", acc[k].data_ptr(), stream=s2.cuda_stream)
+        plan.evaluate("rel32c", stream=s1.cuda_stream)
+    torch.cuda.synchronize()
+    got = acc.cpu().numpy()
+    plan.close()
+    for k in range(8):
+        np.testing.assert_array_equal(got[k], want.astype(np.float32))
+
+
 @pytest.mark.parametrize("ns", [1, 15, 16, 17, 65, 1025])
 def test_direct_sum_sample_sizes(setup, ns):
     """The FP64 direct sum for samples around the sizes of its blocks (16 sinks summed

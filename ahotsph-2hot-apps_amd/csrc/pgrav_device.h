@@ -45,13 +45,15 @@ struct Acc4T {
 typedef Acc4T<float> Acc4;
 
 // -1/sqrt(r2), r2 > 0: v_rsq_f32 in FP32.  In FP64 v_rsq_f64 (relative error <= 5.3e-8)
-// and one third-order step, y + y e (1/2 + 3/8 e) with e = 1 - r2 y^2: six instructions
+// and one third-order step, y + y e (1/2 + 3/8 e) with e = 1 - r2 y^2: seven instructions
 // where a correctly rounded square root and a divide take ~35, and no less exact (largest
 // error over 2^20 values 1.4e-16, mean 4.5e-17; 1/sqrt(r2): 1.7e-16, 5.5e-17).
+// At r2 = 0 and infinity, where e is not a number, the minimum makes it 1 and the result
+// v_rsq_f64's own, -infinity and -0: a source too far for its r2 pulls with nothing.
 __device__ __forceinline__ float nrsq(float r2) { return -__builtin_amdgcn_rsqf(r2); }
 __device__ __forceinline__ double nrsq(double r2) {
     const double y = -__builtin_amdgcn_rsq(r2);
-    const double e = fma(-(r2 * y), y, 1.0);
+    const double e = fmin(fma(-(r2 * y), y, 1.0), 1.0);
     return fma(y * e, fma(0.375, e, 0.5), y);
 }
 

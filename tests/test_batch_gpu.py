@@ -373,6 +373,29 @@ def test_results_stay_whole_under_the_next_evaluation(gpu_lib):
         np.testing.assert_array_equal(got[k], want.astype(np.float32))
 
 
+@pytest.mark.parametrize("soft,eps", [("plummer", 1e-3), ("k1", 1e-3), ("none", 0.0)])
+def test_fp64_source_beyond_the_range_of_its_square(gpu_lib, soft, eps):
+    """A body so far that the FP64 square of its distance is infinite pulls with nothing,
+    in the direct sum and in the batched and per-group FP64 kernels: the other bodies'
+    results are those of a plan without it, up to the order of 48 terms."""
+    from pgrav import batch
+    rng = np.random.default_rng(6)
+    pos = np.concatenate([rng.uniform(size=(48, 3)), [[3e154, 0.0, 0.0]]])
+    mass = np.full(49, 1.0 / 49)
+    got, want = [], []
+    for out, n in ((got, 49), (want, 48)):
+        plan = batch.Plan(pos[:n], mass[:n], order=0, pcut=1000, soft=soft, eps=eps, group_max=48)
+        out.append(plan.direct(np.arange(n)))
+        for v in ("f64", "plain64"):
+            plan.evaluate(v)
+            out.append(plan.result(v))
+        plan.close()
+    scale = np.abs(want[0]).max()
+    for a, b in zip(got, want):
+        np.testing.assert_allclose(a[:48], b, rtol=0, atol=1e-13 * scale)
+        np.testing.assert_array_equal(a[48, :3], np.zeros(3))
+
+
 @pytest.mark.parametrize("ns", [1, 15, 16, 17, 65, 1025])
 def test_direct_sum_sample_sizes(setup, ns):
     """The FP64 direct sum for samples around the sizes of its blocks (16 sinks summed

@@ -4,7 +4,8 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
-#define NXCD 8      // MI355X accelerator complex dies (one L2 each)
+#include "pgrav_grid.h"
+
 #define COUNTER_STRIDE 32  // ints between the persistent launch's work counters: a line each
 
 namespace pgrav {

@@ -836,39 +836,14 @@ hipError_t launch_ewald_table(double L, double *t64, float *t32, hipStream_t st)
     return hipGetLastError();
 }
 
-// Waves that share one group's lists, as a power of two.  A group's lists are a
-// serial chain of LDS tiles and scalar record loads: a wave alone on its SIMD runs
-// at its latency (1 us per order-4 cell), and a launch of a few groups per wave slot
-// ends in a tail of long lists.  Four waves cost nothing where there are many groups;
-// eight and sixteen pay while the groups are few.  us per evaluation by 1, 2, 4, 8, 16
-// waves a group (order 4, theta 0.6 unless stated; in brackets: passes of two plans in
-// turn on two streams, where the tails overlap), every cell in pairs and before the
-// persistent launch's counters had a line each, which took sixteen waves to 33 us in the
-// first row and 122 in the second:
-//   111 groups (Plummer 4,099)            985   486   241   124    65
-//   1,469 (Plummer 65,536, order 2)      1049   525   280   178   143
-//   4,100 (lattice 64^3, images)         2054  1332  1176  1150  1139 [1713 .. 1051 1061 1073]
-//   4,110 (clustered 262,144, FP64)      2217  1735  1367  1281  1348 [1572 .. 1166 1173 1267]
-//   16,457 (clustered 1 M, tolerance)    2012  1613  1333  1246  1300 [1399 .. 1165 1151 1229]
-//   25,034 (clustered 1 M)               3247  2895  2591  2527  2678 [2605 .. 2401 2421 2585]
-//   32,795 (lattice 128^3, Ewald)        5562  5167  4956  5130  5121 [4928 .. 4779 5027 5037]
-//   263,505 (clustered 16.8 M), ms       42.4  42.0  41.2  41.6  44.0 [40.5 .. 40.3 41.9 45.2]
-static int split_log2(int ngroups, int wave_slots) {
-    if (ngroups < wave_slots / 2)
-        return 4;
-    return ngroups < 4 * wave_slots ? 3 : 2;
-}
-
 template <typename T, bool REL, bool COMP, int SOFT, int PER, int BU, int TILE = 64>
 static void launch_one(BatchArgs A, int persistent_blocks, hipStream_t st) {
     // a workgroup's LDS stays within 64 KB (the Ewald terms take 5 or 10 KB a wave)
     while (A.lw && (sizeof(WaveShared<T, PER, TILE>) << A.lw) > 65536) A.lw--;
     const int waves = 1 << A.lw;
     const unsigned lds = (unsigned)(waves * sizeof(WaveShared<T, PER, TILE>));
-    if (persistent_blocks > 0) {
-        // persistent_blocks counts waves; every XCD needs workgroups to drain its slice,
-        // so round up to a multiple of NXCD
-        const int grid = ((persistent_blocks + waves - 1) / waves + NXCD - 1) / NXCD * NXCD;
+    if (persistent_blocks) {
+        const int grid = persistent_grid(persistent_blocks, A.ngroups, waves);
         hipLaunchKernelGGL((k_batch_persistent<T, REL, COMP, SOFT, PER, BU, TILE>), dim3(grid),
                            dim3(64 * waves), lds, st, A, A.bpos, A.cpos, (const T *)A.mom, A.gfirst,
                            A.gcount, A.gcen, A.lpt, A.xoff, A.off, A.idx, (V4<T> *)A.out,
@@ -963,6 +938,8 @@ hipError_t launch_batch(const BatchView &v, int variant, int persistent_blocks, 
             return e;
     }
     A.lw = split_log2(v.ngroups, v.wave_slots);
+    if (persistent_blocks < 0)
+        persistent_blocks = -v.wave_slots;
     if (A.ngroups <= 0)
         return hipSuccess;
     if (v.periodic < 0 || v.periodic > 2 || (v.periodic == 2 && !v.img))

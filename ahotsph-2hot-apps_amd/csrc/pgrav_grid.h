@@ -1,0 +1,41 @@
+// The batched launches' shapes.  No HIP dependency: host tests compile the same rules.
+#pragma once
+
+#define NXCD 8      // MI355X accelerator complex dies (one L2 each)
+
+namespace pgrav {
+
+// Waves that share one group's lists, as a power of two.  A group's lists are a
+// serial chain of LDS tiles and scalar record loads: a wave alone on its SIMD runs
+// at its latency (1 us per order-4 cell), and a launch of a few groups per wave slot
+// ends in a tail of long lists.  Four waves cost nothing where there are many groups;
+// eight and sixteen pay while the groups are few.  us per evaluation by 1, 2, 4, 8, 16
+// waves a group (order 4, theta 0.6 unless stated; in brackets: passes of two plans in
+// turn on two streams, where the tails overlap), every cell in pairs and before the
+// persistent launch's counters had a line each, which took sixteen waves to 33 us in the
+// first row and 122 in the second:
+//   111 groups (Plummer 4,099)            985   486   241   124    65
+//   1,469 (Plummer 65,536, order 2)      1049   525   280   178   143
+//   4,100 (lattice 64^3, images)         2054  1332  1176  1150  1139 [1713 .. 1051 1061 1073]
+//   4,110 (clustered 262,144, FP64)      2217  1735  1367  1281  1348 [1572 .. 1166 1173 1267]
+//   16,457 (clustered 1 M, tolerance)    2012  1613  1333  1246  1300 [1399 .. 1165 1151 1229]
+//   25,034 (clustered 1 M)               3247  2895  2591  2527  2678 [2605 .. 2401 2421 2585]
+//   32,795 (lattice 128^3, Ewald)        5562  5167  4956  5130  5121 [4928 .. 4779 5027 5037]
+//   263,505 (clustered 16.8 M), ms       42.4  42.0  41.2  41.6  44.0 [40.5 .. 40.3 41.9 45.2]
+constexpr int split_log2(int ngroups, int wave_slots) {
+    if (ngroups < wave_slots / 2)
+        return 4;
+    return ngroups < 4 * wave_slots ? 3 : 2;
+}
+
+// Workgroups of a persistent launch, `waves` waves each: as many as asked for, but no more
+// than there are groups, or (negative) those of -blocks waves; a multiple of NXCD, because
+// every XCD needs workgroups to drain its slice.  (Counted in waves, a grid of 256 was 32
+// workgroups of 8 waves on 32 CUs: FP64 on 5,630 groups 8.0 ms, where 256 workgroups of one
+// wave, on a CU each, had taken 6.8.)
+constexpr int persistent_grid(int blocks, int ngroups, int waves) {
+    const int grid = blocks < 0 ? (waves - 1 - blocks) / waves : blocks < ngroups ? blocks : ngroups;
+    return (grid - 1) / NXCD * NXCD + NXCD;
+}
+
+}  // namespace pgrav

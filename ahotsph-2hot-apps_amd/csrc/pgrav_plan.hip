@@ -273,10 +273,7 @@ static int evaluate(Plan *P, int variant, hipStream_t st) {
         fail("unknown variant %d", variant);
         return -1;
     }
-    int pb = P->prm.persistent_blocks;
-    if (pb < 0)
-        pb = P->v.wave_slots;
-    if (!check(launch_batch(P->v, variant, pb, st), "batched kernel"))
+    if (!check(launch_batch(P->v, variant, P->prm.persistent_blocks, st), "batched kernel"))
         return -1;
     return far_field(P, variant, st);
 }
@@ -301,7 +298,7 @@ void pgrav_params_default(pgrav_params *p) {
     p->box = 1.0;
     p->nthreads = 0;
     p->merge_groups = 1;
-    p->persistent_blocks = -1;  // persistent grid, 32 workgroups per CU
+    p->persistent_blocks = -1;  // persistent grid, 32 waves per CU
     p->fp64 = 1;
     p->dispatch = 2;
     p->mixed_order = 0;

@@ -5,8 +5,7 @@ physics: how sink groups are formed (tree cells with siblings merged, then
 optionally merged further where the joint list costs less, or cells cut into
 balanced groups by coordinate bisection), the group size
 (lanes per wave used), the leaf size, the launch shape (one workgroup per group in
-longest-first order, or a persistent grid of k single-wave workgroups per CU
-draining a work counter), the group order inside the per-XCD slices, and the
+longest-first order, or a persistent grid of workgroups draining work counters), the group order inside the per-XCD slices, and the
 unroll factor of the kernel's order-0 and body loops and the tile of list
 entries staged in LDS per round (compiled variants).  The opening angle, multipole order and softening are inputs, so the
 accuracy target is held fixed.  Each candidate is timed with HIP events over
@@ -40,10 +39,9 @@ UNROLL_TILE = [(2, 64), (4, 64), (8, 64), (4, 32), (4, 128)]
 # group order inside the per-XCD slices: 1 longest-first, 2 Morton order (a
 # plan-level choice, no rebuild)
 DISPATCH = [1, 2]
-# launch shapes: 0 = one workgroup per group; -1 = persistent grid of 32
-# single-wave workgroups per CU; k > 0 = persistent grid of k per CU.  The
-# table and tuned.json store the resulting workgroup count (what
-# pgrav_plan_set_launch and Plan(persistent_blocks=...) take).
+# launch shapes, as pgrav_plan_set_launch and Plan(persistent_blocks=...) take them: 0 =
+# one workgroup per group; -1 = a persistent grid of 32 waves per CU; k > 0 = a
+# persistent grid of k workgroups.
 PERSISTENT = [0, -1]
 TUNED = os.path.join(os.path.dirname(os.path.dirname(os.path.abspath(__file__))), "tuned.json")
 

@@ -1,0 +1,35 @@
+"""The batched launches' shapes (csrc/pgrav_grid.h, compiled for the host): a persistent grid
+counts workgroups as asked for and covers every XCD."""
+import os
+import subprocess
+
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+
+PROGRAM = """
+#include <cstdio>
+#include <initializer_list>
+#include "pgrav_grid.h"
+using namespace pgrav;
+int main() {
+    for (int groups : {1, 7, 8, 9, 4095, 4096, 32767, 32768, 1 << 20})
+        for (int blocks : {-8192, 1, 8, 9, 256, 2048, 2147483647}) {
+            const int waves = 1 << split_log2(groups, 8192);
+            printf("%d %d %d %d\\n", groups, blocks, waves, persistent_grid(blocks, groups, waves));
+        }
+}
+"""
+
+
+def test_launch_shapes(tmp_path):
+    (tmp_path / "shape.cpp").write_text(PROGRAM)
+    exe = str(tmp_path / "shape")
+    subprocess.run(["g++", "-std=c++17", "-Wall", "-Werror", "-I",
+                    os.path.join(ROOT, "ahotsph-2hot-apps_amd", "csrc"), str(tmp_path / "shape.cpp"), "-o", exe],
+                   check=True)
+    out = subprocess.run([exe], check=True, capture_output=True, text=True).stdout
+    rows = [[int(x) for x in line.split()] for line in out.splitlines()]
+    assert len(rows) == 9 * 7
+    for groups, blocks, waves, grid in rows:
+        asked = 8192 // waves if blocks < 0 else min(blocks, groups)
+        assert grid == -(-asked // 8) * 8, (groups, blocks, waves, grid)
+        assert waves == (16 if groups < 4096 else 8 if groups < 32768 else 4)

@@ -23,6 +23,9 @@ namespace pgrav {
 //   32,795 (lattice 128^3, Ewald)        5562  5167  4956  5130  5121 [4928 .. 4779 5027 5037]
 //   263,505 (clustered 16.8 M), ms       42.4  42.0  41.2  41.6  44.0 [40.5 .. 40.3 41.9 45.2]
 constexpr int split_log2(int ngroups, int wave_slots) {
+    // (a launch holds fewer than 2^32 lanes, and its workgroups are rounded up to NXCD)
+    if (ngroups > (1 << 24) - NXCD)
+        return ngroups > (1 << 25) - NXCD ? 0 : 1;
     if (ngroups < wave_slots / 2)
         return 4;
     return ngroups < 4 * wave_slots ? 3 : 2;

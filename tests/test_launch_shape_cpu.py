@@ -1,5 +1,5 @@
 """The batched launches' shapes (csrc/pgrav_grid.h, compiled for the host): a persistent grid
-counts workgroups as asked for and covers every XCD."""
+counts workgroups as asked for, covers every XCD, and no launch exceeds 2^32 - 1 lanes."""
 import os
 import subprocess
 
@@ -11,7 +11,8 @@ PROGRAM = """
 #include "pgrav_grid.h"
 using namespace pgrav;
 int main() {
-    for (int groups : {1, 7, 8, 9, 4095, 4096, 32767, 32768, 1 << 20})
+    for (int groups : {1, 7, 8, 9, 4095, 4096, 32767, 32768, 1 << 20, (1 << 24) - 8, (1 << 24) - 7,
+                       1 << 24, (1 << 25) - 8, (1 << 25) - 7, 1 << 25, (1 << 26) - 8})
         for (int blocks : {-8192, 1, 8, 9, 256, 2048, 2147483647}) {
             const int waves = 1 << split_log2(groups, 8192);
             printf("%d %d %d %d\\n", groups, blocks, waves, persistent_grid(blocks, groups, waves));
@@ -28,8 +29,10 @@ def test_launch_shapes(tmp_path):
                    check=True)
     out = subprocess.run([exe], check=True, capture_output=True, text=True).stdout
     rows = [[int(x) for x in line.split()] for line in out.splitlines()]
-    assert len(rows) == 9 * 7
+    assert len(rows) == 16 * 7
     for groups, blocks, waves, grid in rows:
         asked = 8192 // waves if blocks < 0 else min(blocks, groups)
         assert grid == -(-asked // 8) * 8, (groups, blocks, waves, grid)
-        assert waves == (16 if groups < 4096 else 8 if groups < 32768 else 4)
+        assert max(groups, grid) * 64 * waves < 2 ** 32, (groups, blocks, waves, grid)
+        assert waves == (16 if groups < 4096 else 8 if groups < 32768 else 4 if groups < 2 ** 24 - 7 else
+                         2 if groups < 2 ** 25 - 7 else 1)

@@ -20,6 +20,9 @@ constexpr double FAR_ETA = 1e-4;
 // Lists a wave would not fill once stay in pairs; a group with fewer cells has no expansion
 // (its sums over the lanes and its evaluation cost as much as ~30 order-4 cells).
 constexpr int FAR_MIN_LIST = 32, FAR_MIN_CELLS = 64;
+// The coefficients' unit of length is the sinks' radius, in FP32: below this a cell's first
+// degrees, mass / d (radius / d)^l, and the radius itself leave its range.
+constexpr double FAR_MIN_RADIUS = 1e-20;
 
 // a list entry's position: bodies and cells, at the image (i, j, k) of nln/mac.c:91-111
 // where lists carry one

@@ -115,8 +115,10 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2))) void k_
     double rs2 = sx * sx + sy * sy + sz * sz;
     for (int h = 32; h > 0; h >>= 1) rs2 = fmax(rs2, __shfl_xor(rs2, h));
     const double rs = sqrt(rs2);
-    // sinks outside the sphere that says which image they see (moved bodies): no expansion
-    const bool off = ncell < FAR_MIN_CELLS || !(rs > 0.0) || (PER == 1 && rs > gc.w * (1.0 + 1e-9));
+    // sinks all but at one point, or outside the sphere that says which image they see (moved
+    // bodies): no expansion
+    const bool off = ncell < FAR_MIN_CELLS || !(rs > FAR_MIN_RADIUS) ||
+                     (PER == 1 && rs > gc.w * (1.0 + 1e-9));
     const double far2 = off ? (double)INFINITY
                             : fmax(rs2 / (FAR_RHO * FAR_RHO), SOFT ? A.eps * A.eps / FAR_ETA : 0.0);
     if (lane == 0)

@@ -350,6 +350,26 @@ def test_far_cells_match_the_pairs(gpu_lib, kw):
     plan.close()
 
 
+@pytest.mark.parametrize("size", [0.0, 1e-44, 1e-41, 1e-30, 1e-19, 1e-9])
+def test_far_cells_of_a_vanishing_group(gpu_lib, size):
+    """Eight bodies closer to one another than FP32 can tell, in a group of their own, among
+    many: their results against FP64's (a few 1e-7 of the pulls' sum, as above)."""
+    from pgrav import batch, ics
+    pos, mass = ics.clustered(60000, seed=21, nhalo=24)
+    pos = (pos - pos.min(0)) / (np.ptp(pos, 0).max() * 1.001)
+    pos = np.concatenate([pos + 0.001, size * np.arange(8.0)[:, None] * [[1.0, 0.5, 0.25]]])
+    plan = batch.Plan(pos, np.append(mass, np.full(8, mass[0])), theta=0.4, order=4, eps=1e-3,
+                      group_max=8, leaf_max=16)
+    assert _far_pays(plan.stats(), False)
+    plan.evaluate("f64")
+    ref = plan.result("f64")[-8:]
+    for var in ("rel32c", "rel32"):
+        plan.evaluate(var)
+        got = plan.result(var)[-8:]
+        np.testing.assert_allclose(got, ref, rtol=0, atol=3e-6 * np.abs(ref[:, :3]).max())
+    plan.close()
+
+
 def test_results_stay_whole_under_the_next_evaluation(gpu_lib):
     """A result read on one stream while the same bodies are evaluated again on another:
     the result array holds whole sums only, so every read gives the first one's values."""

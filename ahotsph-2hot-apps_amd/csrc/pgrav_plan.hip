@@ -166,10 +166,17 @@ static int device_wave_slots() {
 //   order 0, 1 M (26,465, 813)        870  945    tolerance 1 M (16,454, 47 + 22 + 1,704) 1272 1378
 //   Ewald 64^3 (4,102, 794)          1241 1294    Ewald 96^3 (16,384, 794) 3617 3387
 //   Ewald 128^3 (32,795, 910)        5281 4014
+// Groups of one body have no expansion and leave k_far at once; where all are (400,000
+// bodies), 22.3 ms a pass without it and 22.6 with it.
 static bool far_pays(const Lists &L, int wave_slots, int periodic) {
-    const int64_t G = L.ngroups;
-    return 38 * L.off[L_HEXA].back() + 8 * L.off[L_QUAD].back() >
-               6500 * G + (int64_t)4000 * wave_slots &&
+    int64_t G = 0, hexa = 0, quad = 0;
+    for (int64_t g = 0; g < L.ngroups; g++)
+        if (L.gcount[g] > 1) {
+            G++;
+            hexa += L.off[L_HEXA][g + 1] - L.off[L_HEXA][g];
+            quad += L.off[L_QUAD][g + 1] - L.off[L_QUAD][g];
+        }
+    return 38 * hexa + 8 * quad > 6500 * G + (int64_t)4000 * wave_slots &&
            (periodic != 1 || G >= 2 * (int64_t)wave_slots);
 }
 

@@ -12,6 +12,7 @@
 #include <cmath>
 #include <new>
 #include <stdexcept>
+#include <type_traits>
 #include <vector>
 
 #include "../../include/pgrav.h"
@@ -73,6 +74,26 @@ struct Plan {
             throw std::runtime_error("device allocation failed");
         allocs.push_back(p);
         return (P *)p;
+    }
+    // The local expansions' workspace (pgrav_far.hip): the far cells' pull and what is left of
+    // the cell lists.  Where the memory ends here it is left out, and every cell is taken in
+    // pairs.
+    void far_alloc(int64_t cells) {
+        const size_t mark = allocs.size(), G = v.ngroups;
+        auto get = [&](auto *&out, size_t count) {
+            void *p = nullptr;
+            if (hipMalloc(&p, count * sizeof(*out)) != hipSuccess)
+                return false;
+            allocs.push_back(p);
+            out = (std::remove_reference_t<decltype(out)>)p;
+            return true;
+        };
+        if (get(v.far2, G) && get(v.far_pull, 2 * (size_t)tree.n) && get(v.near_n, 3 * G) &&
+            get(v.near, cells) && (prm.periodic != 2 || get(v.near_img, cells)))
+            return;
+        (void)hipGetLastError();  // (not a later launch's)
+        v.far2 = nullptr;
+        for (; allocs.size() > mark; allocs.pop_back()) (void)hipFree(allocs.back());
     }
     template <typename P>
     P *upload(const P *h, size_t count) {
@@ -453,18 +474,6 @@ void *pgrav_plan_create(const double *pos3, const double *mass, int64_t n, const
         P->v.out32 = P->dalloc<float4>(sizeof(float4) * (size_t)n);
         if (p->fp64)
             P->v.out64 = P->dalloc<double4>(sizeof(double4) * (size_t)n);
-        if (far_pays(L, P->v.wave_slots, p->periodic)) {
-            // the local expansions' workspace: the far cells' pull and the rest of the lists
-            const size_t G = std::max(1, P->v.ngroups);
-            int64_t cells = 0;
-            for (int k = 0; k < L_BODY; k++) cells += L.off[k].back();
-            P->v.far2 = P->dalloc<double>(sizeof(double) * G);
-            P->v.far_pull = P->dalloc<float4>(2 * sizeof(float4) * (size_t)n);
-            P->v.near_n = P->dalloc<int>(sizeof(int) * 3 * G);
-            P->v.near = P->dalloc<uint32_t>(sizeof(uint32_t) * cells);
-            if (p->periodic == 2)
-                P->v.near_img = P->dalloc<uint8_t>(cells);
-        }
         const size_t cbytes = sizeof(int) * COUNTER_STRIDE * (2 + NXCD);
         P->v.counter = P->dalloc<int>(cbytes);
         if (!check(hipMemset(P->v.counter, 0, cbytes), "hipMemset"))
@@ -496,6 +505,8 @@ void *pgrav_plan_create(const double *pos3, const double *mass, int64_t n, const
             P->v.ewald32 = t32;
             P->v.ewald64 = t64;
         }
+        if (far_pays(L, P->v.wave_slots, p->periodic))
+            P->far_alloc(L.off[L_HEXA].back() + L.off[L_QUAD].back() + L.off[L_MONO].back());
         if (!check(hipStreamSynchronize(P->stream), "hipStreamSynchronize"))
             throw std::runtime_error("sync");
         P->t_upload = now() - t2;

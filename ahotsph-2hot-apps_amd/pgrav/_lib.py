@@ -108,10 +108,13 @@ def check():
 def ptr(a):
     """Raw pointer of a numpy array (or None).  Through the buffer protocol: numpy's own
     a.ctypes.data costs 2.5 us, more than most drop-in calls; it serves the arrays whose
-    buffer ctypes does not take (read-only, empty, not C-contiguous)."""
+    buffer ctypes does not take (read-only, empty, not C-contiguous) and refuses what is
+    no array, which may well have a buffer."""
     if a is None:
         return None
-    try:
-        return ctypes.c_void_p(ctypes.addressof(ctypes.c_char.from_buffer(a)))
-    except (TypeError, ValueError, BufferError):
-        return ctypes.c_void_p(a.ctypes.data)
+    if isinstance(a, np.ndarray):
+        try:
+            return ctypes.c_void_p(ctypes.addressof(ctypes.c_char.from_buffer(a)))
+        except (TypeError, ValueError, BufferError):
+            pass
+    return ctypes.c_void_p(a.ctypes.data)

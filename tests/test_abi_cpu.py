@@ -106,3 +106,21 @@ print("DONE")
     assert lines[-1] == "DONE"
     assert "NOERR" not in r.stdout, r.stdout
     assert any(l.startswith("ERR") for l in lines)
+
+
+def test_array_pointers():
+    """ptr() gives an array's own address in every layout, and takes arrays only: objects
+    with a buffer of their own (bytes, memory views) are no float tables."""
+    import array
+
+    import numpy as np
+    from pgrav._lib import ptr
+    a = np.arange(24, dtype=np.float32).reshape(4, 6)
+    fixed = a.copy()
+    fixed.flags.writeable = False
+    for x in (a, a[1:], a[:, 2:], a.T, a[::-1], fixed, np.empty((0, 3)), np.array(1.5)):
+        assert ptr(x).value == (x.ctypes.data or None)
+    assert ptr(None) is None
+    for x in (bytearray(8), memoryview(bytearray(8)), array.array("f", [1.0]), b"abcd", [1.0], 1.0):
+        with pytest.raises(AttributeError):
+            ptr(x)

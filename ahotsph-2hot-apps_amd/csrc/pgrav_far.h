@@ -8,13 +8,20 @@
 namespace pgrav {
 
 // A cell is far when the group's sinks reach less than FAR_RHO of its distance from the
-// group centre and (eps / distance)^2 is below FAR_ETA.  The expansion's first term left
-// out is then at most 9 FAR_RHO^8 = 6e-6 of the cell's pull, at the outermost sink and
-// for the nearest far cell; over all sinks the error against the FP64 evaluation of the
-// same lists is below that of the pairs alone: median |da|/|a| 6.8e-8 (pairs 9.8e-8),
-// 99th percentile 5.2e-7 (5.8e-7) at 1 M clustered bodies; on the 64^3 lattice of
-// explicit images 1.6e-5 (5.3e-5) and 9e-5 (3.1e-4).  0.25 gains 3 % and triples the
-// 99th percentile.
+// group centre and (eps / distance)^2 is below FAR_ETA.  At the outermost sink and for the
+// nearest far cell the degrees left out are then 7.7e-6 of a point's pull; a cell's moment
+// of order k brings them with a factor (l + k)! / (k! l!) (extent / distance)^k, so that a
+// cell of two bodies 0.2, 0.4, 0.5 of its distance from their mean is at worst 2.6e-5,
+// 7.9e-5, 1.2e-4 of m / d^2 off at order 2 and 3.5e-5, 2.3e-4, 5.0e-4 at order 4 (which
+// itself leaves out the cell's order 5, (extent / distance)^5).  Most far cells are much
+// farther and rounder: over all sinks the error against the FP64 evaluation of the same
+// lists is below that of the pairs alone: median |da|/|a| 6.9e-8 (pairs 1.0e-7), 99th
+// percentile 4.7e-7 (5.5e-7), largest 4.7e-6 of the rms pull (4.7e-6) at 1 M clustered
+// bodies; on the 64^3 lattice of explicit images 1.6e-5 (5.3e-5), 9e-5 (3.1e-4), 4.9e-5
+// (2.1e-4); over 70 plans of 30,000 to 700,000 bodies (orders, softenings, angles, periodic
+// schemes) the 2-norm of the error is 0.8 of the pairs' in the mean and 1.002 at most, the
+// largest error 1.16 at most.  0.25 gains 3 % and triples the 99th percentile; 0.15 costs
+// 1.5 to 3 % (16.8 M 27.1 ms, images 64^3 813 us instead of 26.6 and 783), 0.13 3 to 8 %.
 constexpr double FAR_RHO = 0.17;
 constexpr double FAR_ETA = 1e-4;
 // Lists a wave would not fill once stay in pairs; a group with fewer cells has no expansion

@@ -175,8 +175,9 @@ constexpr LxAxial lx_make_axial() {
     return r;
 }
 constexpr LxAxial LX_AX = lx_make_axial();
-constexpr int LX_SOFT_L = 5;  // degrees whose softening terms are kept: at (eps/d)^2 <= LX_ETA
-                              // and r_s < 0.17 d the others are below 1e-8 of the cell's pull
+constexpr int LX_SOFT_L = 5;  // degrees whose softening terms are kept: of a point, at (eps / d)^2
+                              // = FAR_ETA and r_s = FAR_RHO d (pgrav_far.h), degree 6's is 2.6e-7
+                              // of the pull and 7's 6e-8
 
 template <typename T>
 PGRAV_HD inline T lx_rsqrt(T x) {

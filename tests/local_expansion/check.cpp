@@ -35,43 +35,99 @@ void field(const double *M, int order, const double *X, double eps2, double *out
     }
 }
 
-// a cell of points at c (about their mean): its prepared record through traceless moments
-void cell(std::mt19937_64 &g, double size, int order, double *M) {
-    std::uniform_real_distribution<double> U(-0.5, 0.5);
-    const int n = 20;
-    std::vector<std::array<double, 3>> p(n);
+// the prepared record of points about their mean, of masses m (sum 1), through traceless moments
+void record(const std::vector<std::array<double, 3>> &points, const std::vector<double> &m, double size,
+            int order, double *M) {
+    std::vector<std::array<double, 3>> p = points;
+    const int n = (int)p.size();
     double mean[3] = {0, 0, 0};
-    for (auto &q : p)
-        for (int k = 0; k < 3; k++) mean[k] += (q[k] = size * U(g)) / n;
+    for (int i = 0; i < n; i++)
+        for (int k = 0; k < 3; k++) mean[k] += m[i] * p[i][k];
     double q[29] = {0};
     q[0] = 1;
     q[4] = size;
     auto dl = [](int i, int j) { return i == j ? 1.0 : 0.0; };
-    for (auto &b : p) {
+    for (int i0 = 0; i0 < n; i0++) {
         double x[3], r2 = 0;
-        for (int k = 0; k < 3; k++) r2 += (x[k] = (b[k] - mean[k]) / size) * x[k];
+        for (int k = 0; k < 3; k++) {
+            x[k] = (p[i0][k] - mean[k]) / size;
+            r2 += x[k] * x[k];
+        }
         const int i2[5][2] = {{0, 0}, {0, 1}, {1, 1}, {0, 2}, {1, 2}};
         const int i3[7][3] = {{0, 0, 0}, {0, 0, 1}, {0, 1, 1}, {1, 1, 1}, {0, 0, 2}, {0, 1, 2}, {1, 1, 2}};
         const int i4[9][4] = {{0, 0, 0, 0}, {0, 0, 0, 1}, {0, 0, 1, 1}, {0, 1, 1, 1}, {1, 1, 1, 1},
                               {0, 0, 0, 2}, {0, 0, 1, 2}, {0, 1, 1, 2}, {1, 1, 1, 2}};
         for (int t = 0; t < 5; t++) {
             const int i = i2[t][0], j = i2[t][1];
-            q[8 + t] += (x[i] * x[j] - r2 / 3 * dl(i, j)) / n;
+            q[8 + t] += m[i0] * (x[i] * x[j] - r2 / 3 * dl(i, j));
         }
         for (int t = 0; t < 7; t++) {
             const int i = i3[t][0], j = i3[t][1], l = i3[t][2];
-            q[13 + t] += (x[i] * x[j] * x[l] -
-                          r2 / 5 * (dl(i, j) * x[l] + dl(i, l) * x[j] + dl(j, l) * x[i])) / n;
+            q[13 + t] += m[i0] * (x[i] * x[j] * x[l] -
+                                  r2 / 5 * (dl(i, j) * x[l] + dl(i, l) * x[j] + dl(j, l) * x[i]));
         }
         for (int t = 0; t < 9; t++) {
-            const int i = i4[t][0], j = i4[t][1], l = i4[t][2], m = i4[t][3];
-            q[20 + t] += (x[i] * x[j] * x[l] * x[m] -
-                          r2 / 7 * (dl(i, j) * x[l] * x[m] + dl(i, l) * x[j] * x[m] + dl(i, m) * x[j] * x[l] +
-                                    dl(j, l) * x[i] * x[m] + dl(j, m) * x[i] * x[l] + dl(l, m) * x[i] * x[j]) +
-                          r2 * r2 / 35 * (dl(i, j) * dl(l, m) + dl(i, l) * dl(j, m) + dl(i, m) * dl(j, l))) / n;
+            const int i = i4[t][0], j = i4[t][1], l = i4[t][2], k = i4[t][3];
+            q[20 + t] += m[i0] *
+                         (x[i] * x[j] * x[l] * x[k] -
+                          r2 / 7 * (dl(i, j) * x[l] * x[k] + dl(i, l) * x[j] * x[k] + dl(i, k) * x[j] * x[l] +
+                                    dl(j, l) * x[i] * x[k] + dl(j, k) * x[i] * x[l] + dl(l, k) * x[i] * x[j]) +
+                          r2 * r2 / 35 * (dl(i, j) * dl(l, k) + dl(i, l) * dl(j, k) + dl(i, k) * dl(j, l)));
         }
     }
     prep_record<double>(q, order, 0, M);
+}
+
+// a cell of 20 points of one mass, anywhere in a box
+void cell(std::mt19937_64 &g, double size, int order, double *M) {
+    std::uniform_real_distribution<double> U(-0.5, 0.5);
+    std::vector<std::array<double, 3>> p(20);
+    for (auto &q : p)
+        for (int k = 0; k < 3; k++) q[k] = size * U(g);
+    record(p, std::vector<double>(20, 0.05), size, order, M);
+}
+
+// One cell of two points at distance at most b from their mean, anywhere around the group
+// and turned any way: the largest error in units of the cell's pull as a point, m / d^2.
+template <int ORDER>
+void run_two(double rho, double bd) {
+    std::mt19937_64 g(2);
+    std::normal_distribution<double> N;
+    double worst = 0;
+    for (int c = 0; c < 400; c++) {
+        auto unit = [&](double *n) {
+            double r = 0;
+            for (int k = 0; k < 3; k++) {
+                n[k] = N(g);
+                r += n[k] * n[k];
+            }
+            for (int k = 0; k < 3; k++) n[k] /= sqrt(r);
+        };
+        double n[3], t[3];
+        unit(n);
+        unit(t);
+        if (c < 100)  // along the line of sight
+            for (int k = 0; k < 3; k++) t[k] = c % 2 ? n[k] : -n[k];
+        const double f = 0.5 + 0.1 * (c % 5);  // the share of the point nearer to the mean
+        double M[PREC4];
+        record({{t[0] * bd, t[1] * bd, t[2] * bd},
+                {-t[0] * bd * (1 - f) / f, -t[1] * bd * (1 - f) / f, -t[2] * bd * (1 - f) / f}},
+               {1 - f, f}, bd, ORDER, M);
+        std::vector<double> A(LX_ALL, 0.0);
+        lx_add_cell<ORDER, false, double>(M, 1.0, n[0], n[1], n[2], 0.0, rho, A.data());
+        for (int i = 0; i < 64; i++) {
+            double u[3], o[4], r[4] = {0, 0, 0, 0}, e = 0;
+            unit(u);
+            if (i < 2)  // towards the cell and away from it
+                for (int k = 0; k < 3; k++) u[k] = i ? n[k] : -n[k];
+            lx_evaluate<false, 0, double>(A.data(), u[0], u[1], u[2], 1 / rho, o);
+            const double X[3] = {rho * u[0] - n[0], rho * u[1] - n[1], rho * u[2] - n[2]};
+            field(M, ORDER, X, 0.0, r);
+            for (int k = 0; k < 3; k++) e += (o[k] - r[k]) * (o[k] - r[k]);
+            worst = std::max(worst, sqrt(e));
+        }
+    }
+    printf("two %d %g %g %.3e\n", ORDER, rho, bd, worst);
 }
 
 template <int ORDER, bool SOFT, typename T>
@@ -143,5 +199,14 @@ int main() {
             run<4, true, float>(rho, eta);
         }
     }
+    for (double rho : {0.05, 0.17})
+        for (double bd : {0.0, 0.2, 0.4, 0.5, 0.6}) {
+            if (bd == 0.0)
+                run_two<0>(rho, 1e-3);
+            else {
+                run_two<2>(rho, bd);
+                run_two<4>(rho, bd);
+            }
+        }
     return 0;
 }

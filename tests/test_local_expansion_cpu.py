@@ -5,7 +5,12 @@ beside the axis of its harmonics.
 The bound: the first degree left out pulls at most 9 rho^8 of a cell's pull at the
 outermost sink (the multipoles and the cells' partial cancellation allow ten times
 that); softening is kept to first order in eta = (eps / d)^2 and to total degree 5, so
-what is left out is of order eta^2 and eta rho^5; FP32 adds its rounding."""
+what is left out is of order eta^2 and eta rho^5; FP32 adds its rounding.
+
+One cell alone can be that much worse: its moment of order k, at most m b^k for bodies
+within b of its centre, brings the degrees l left out with a factor (l + k)! / (k! l!), so
+in units of m / d^2 at most sum_{l > 8} l rho^(l-1) sum_k C(l + k, k) (b / d)^k."""
+import math
 import os
 import subprocess
 
@@ -18,7 +23,7 @@ def test_expansion_matches_the_cells_fields(tmp_path):
                     os.path.join(ROOT, "tests", "local_expansion", "check.cpp"), "-o", str(exe)],
                    check=True)
     lines = subprocess.run([str(exe)], check=True, capture_output=True, text=True).stdout.split("\n")
-    rows = [l.split() for l in lines if l]
+    rows = [l.split() for l in lines if l and not l.startswith("two")]
     assert len(rows) == 54
     for order, soft, size, rho, eta, acc, phi in rows:
         rho, eta = float(rho), float(eta) * int(soft)
@@ -26,3 +31,10 @@ def test_expansion_matches_the_cells_fields(tmp_path):
             (1e-13 if size == "8" else 64 * 2.0 ** -24)
         assert float(acc) < bound, (order, soft, size, rho, eta, acc, bound)
         assert float(phi) < bound, (order, soft, size, rho, eta, phi, bound)
+    two = [[float(x) for x in l.split()[1:]] for l in lines if l.startswith("two")]
+    assert len(two) == 18
+    for order, rho, bd, worst in two:
+        bound = sum(l * rho ** (l - 1) * sum(math.comb(l + k, k) * bd ** k for k in range(int(order) + 1) if k != 1)
+                    for l in range(9, 60))
+        # (printed to four digits; two points on the line of sight reach it at orders 0 and 2)
+        assert 0.6 * bound < worst < 1.001 * bound, (order, rho, bd, worst, bound)

@@ -179,14 +179,18 @@ static int device_wave_slots() {
 // chain cost ~35 us, 4,000 instructions per wave slot.  The Ewald kernel still reads
 // every entry for the correction and gains only with many groups.  us per evaluation in
 // pairs and with expansions (groups, cells listed by each):
-//   clustered 65,536 (1,830, 269)     172  177    Plummer 65,536 (1,452, 667)   283  302
-//   clustered 131,072 (3,679, 353)    340  308    Plummer 262,144 (5,738, 943)  907  668
-//   clustered 524,288 (14,061, 506)  1283 1032    clustered 2 M (32,903, 748)  4500 3555
-//   images 32^3 (512, 1,600)          204  200    images 64^3 (4,102, 1,908)   1197  810
-//   order 2, 1 M (26,465, 773)       1357 1412    order 2 Plummer 262,144 (5,738, 1,109) 479 452
-//   order 0, 1 M (26,465, 813)        870  945    tolerance 1 M (16,454, 47 + 22 + 1,704) 1272 1378
-//   Ewald 64^3 (4,102, 794)          1241 1294    Ewald 96^3 (16,384, 794) 3617 3387
-//   Ewald 128^3 (32,795, 910)        5281 4014
+//   clustered 65,536 (1,830, 269)     156  157    Plummer 65,536 (1,452, 667)   278  301
+//   clustered 131,072 (3,679, 353)    315  285    Plummer 262,144 (5,738, 943)  864  626
+//   clustered 524,288 (14,061, 506)  1226  923    clustered 2 M (32,903, 748)  4218 3055
+//   images 32^3 (512, 1,600)          176  174    images 64^3 (4,102, 1,908)   1131  774
+//   order 2, 1 M (26,465, 773)       1274 1240    order 2 Plummer 262,144 (5,738, 1,109) 434 400
+//   order 0, 1 M (26,465, 813)        821  858    tolerance 1 M (16,454, 47 + 22 + 1,704) 1220 1204
+//   Ewald 64^3 (4,102, 794)          1204 1260    Ewald 96^3 (16,384, 794) 3482 3247
+//   Ewald 128^3 (32,795, 910)        5012 3847
+// The line is on the safe side at clustered 131,072 and at order 2, and blind to what it
+// does not look at, the cells' distances: with softening none nearer than 100 eps is far,
+// and where that leaves none the scan of the lists is lost (clustered 1 M by eps: 1e-4 1821,
+// 1e-3 2095, 1e-2 2831 against 2596 in pairs; Plummer 262,144 at eps 0.1 906 against 868).
 // Groups of one body have no expansion and leave k_far at once; where all are (400,000
 // bodies), 22.3 ms a pass without it and 22.6 with it.
 static bool far_pays(const Lists &L, int wave_slots, int periodic) {

@@ -25,6 +25,9 @@
 // workgroup per group.
 #include <math.h>
 
+#include <algorithm>
+#include <array>
+
 #include "pgrav_batch.h"
 #include "pgrav_device.h"
 #include "pgrav_ewald.h"
@@ -73,6 +76,8 @@ struct BatchArgs {
     int ngroups;
     int soft;
     int lw;  // log2 of the waves that share a group's lists
+    int given;  // persistent launch: how many groups of each slice need no counter
+    int cus;
     double eps;
     double G;
     double box;
@@ -550,11 +555,13 @@ void k_batch_persistent(
     extern __shared__ __align__(16) char smem[];
     __shared__ int w;
     const int x = blockIdx.x % NXCD;
-    // the first groups of each slice are the workgroups' own, without a counter
-    const int given = gridDim.x / NXCD;
-    int item = A.xoff[x] + (int)blockIdx.x / NXCD;
-    bool own = item < A.xoff[x + 1];  // the own slice may have more groups
-    if (!own)
+    // the first groups of each slice are the own ones of the workgroups that are resident
+    // from the start, without a counter (a group given to one that has to wait for a place
+    // would be taken when all others are done: FP64 Ewald 64^3 2,948 us, so 2,846)
+    const int given = A.given, mine = blockIdx.x / NXCD;
+    int item = A.xoff[x] + mine;
+    bool own = given < A.xoff[x + 1] - A.xoff[x];  // the own slice may have more groups
+    if (mine >= given || item >= A.xoff[x + 1])
         item = -1;
     for (;;) {
         if (item < 0) {
@@ -843,11 +850,23 @@ static void launch_one(BatchArgs A, int persistent_blocks, hipStream_t st) {
     const int waves = 1 << A.lw;
     const unsigned lds = (unsigned)(waves * sizeof(WaveShared<T, PER, TILE>));
     if (persistent_blocks) {
+        const auto kernel = k_batch_persistent<T, REL, COMP, SOFT, PER, BU, TILE>;
+        // workgroups a CU holds, by the log2 of their waves: a property of the kernel
+        static const std::array<int, 5> held = [&] {
+            std::array<int, 5> n{};
+            for (int w = 0; w < 5 && (sizeof(WaveShared<T, PER, TILE>) << w) <= 65536; w++)
+                if (hipOccupancyMaxActiveBlocksPerMultiprocessor(
+                        &n[w], (const void *)kernel, 64 << w, sizeof(WaveShared<T, PER, TILE>) << w) != hipSuccess) {
+                    (void)hipGetLastError();
+                    n[w] = 0;
+                }
+            return n;
+        }();
         const int grid = persistent_grid(persistent_blocks, A.ngroups, waves);
-        hipLaunchKernelGGL((k_batch_persistent<T, REL, COMP, SOFT, PER, BU, TILE>), dim3(grid),
-                           dim3(64 * waves), lds, st, A, A.bpos, A.cpos, (const T *)A.mom, A.gfirst,
-                           A.gcount, A.gcen, A.lpt, A.xoff, A.off, A.idx, (V4<T> *)A.out,
-                           A.counter, A.ewald);
+        A.given = std::min(grid, held[A.lw] * A.cus) / NXCD;
+        hipLaunchKernelGGL(kernel, dim3(grid), dim3(64 * waves), lds, st, A, A.bpos, A.cpos,
+                           (const T *)A.mom, A.gfirst, A.gcount, A.gcen, A.lpt, A.xoff, A.off, A.idx,
+                           (V4<T> *)A.out, A.counter, A.ewald);
     } else {
         hipLaunchKernelGGL((k_batch<T, REL, COMP, SOFT, PER, BU, TILE>), dim3(A.ngroups),
                            dim3(64 * waves), lds, st, A);
@@ -938,6 +957,8 @@ hipError_t launch_batch(const BatchView &v, int variant, int persistent_blocks, 
             return e;
     }
     A.lw = split_log2(v.ngroups, v.wave_slots);
+    A.given = 0;
+    A.cus = v.wave_slots / 32;
     if (persistent_blocks < 0)
         persistent_blocks = -v.wave_slots;
     if (A.ngroups <= 0)
@@ -990,7 +1011,7 @@ hipError_t launch_group64(const BatchView &v, int g, hipStream_t st) {
     A.near = nullptr;
     A.near_img = nullptr;
     A.near_n = nullptr;
-    A.lw = 0;
+    A.lw = A.given = A.cus = 0;
     if (v.periodic < 0 || v.periodic > 2 || (v.periodic == 2 && !v.img))
         return hipErrorInvalidValue;
     const int per = v.periodic;

@@ -9,6 +9,7 @@ G = 1.  One step = one force evaluation of every body's interaction list (one
 kernel launch) with inputs resident in HBM.  Prints one JSON line.
 """
 import argparse
+import hashlib
 import json
 import os
 import sys
@@ -30,6 +31,32 @@ FLOPS = {"hexa": 217, "quad": 66, "mono": 26, "body": 26}
 # algorithmic bytes per list entry / per sink (prepared FP32 record + FP64 centre)
 BYTES_ENTRY = {"hexa": 4 + 32 + 184, "quad": 4 + 32 + 40, "mono": 4 + 32, "body": 4 + 32}
 BYTES_SINK = 32 + 16
+
+
+# what decides how much an evaluation of given lists issues and moves
+KERNEL_SOURCES = ("pgrav_batch.hip", "pgrav_far.hip", "pgrav_plan.hip", "pgrav_batch.h", "pgrav_device.h",
+                  "pgrav_ewald.h", "pgrav_far.h", "pgrav_grid.h", "pgrav_local.h", "pgrav_record.h")
+
+
+def kernel_sources():
+    h = hashlib.sha256()
+    for name in KERNEL_SOURCES:
+        with open(os.path.join(PKG, "csrc", name), "rb") as f:
+            h.update(f.read())
+    return h.hexdigest()[:16]
+
+
+def profiled(path, key, npairs):
+    """The profile's record of this workload and launch, if it was taken with these lists
+    and these kernels' sources; else None."""
+    try:
+        with open(path) as f:
+            rec = json.load(f).get(key)
+    except (OSError, ValueError):
+        return None
+    if not rec or rec.get("sources") != kernel_sources() or rec.get("pairs") != npairs:
+        return None
+    return rec
 
 
 def log(*a):
@@ -161,7 +188,9 @@ def main():
     npairs = sum(pairs.values())
     flops = sum(FLOPS[k] * pairs[k] for k in FLOPS)
     nbytes = sum(BYTES_ENTRY[k] * st["entries_" + k] for k in FLOPS) + BYTES_SINK * st["n"]
-    achieved = flops / (kern_ms * 1e-3) / 1e12
+    # by the reference's flops of the listed pairs: a rate to compare evaluations of the same
+    # lists by, and more than a kernel issues that takes a group's far cells through one expansion
+    ref_achieved = flops / (kern_ms * 1e-3) / 1e12
 
     # accuracy at this configuration vs the FP64 direct sum on sampled bodies
     rng = np.random.default_rng(12345)
@@ -185,34 +214,16 @@ def main():
         log("plain FP64 one-launch-per-group %.1f ms -> speedup %.1fx" % (plain_ms, plain_ms / kern_ms))
     baselines["speedup_vs_batched_fp64"] = f64_ms / kern_ms
 
-    # HBM bytes per launch of the batched kernel, measured with rocprofv3
-    # FETCH_SIZE / WRITE_SIZE for this exact workload and scaled by the same
-    # counters on a copy of known size (profiles/traffic.json records how)
-    traffic = None
-    try:
-        with open(os.path.join(ROOT, "profiles", "traffic.json")) as f:
-            rec = json.load(f).get(workload_name(args, pos.shape[0], var, dec))
-        if rec:
-            traffic = rec["bytes_per_launch"]
-    except (OSError, ValueError, KeyError):
-        traffic = None
-
-    # FP32 flops the hardware issued per launch for this exact workload and launch
-    # (rocprofv3 SQ_INSTS_VALU_FLOPS_FP32 x 64 lanes; profiles/valu_flops.json
-    # records the run).  Where it is known it is the achieved rate; the reference's
-    # flops of the listed pairs are more than a kernel issues that takes a group's far
-    # cells through one expansion, and give the rate in `reference_achieved`
-    hw_flops = None
-    try:
-        with open(os.path.join(ROOT, "profiles", "valu_flops.json")) as f:
-            rec = json.load(f).get(workload_name(args, pos.shape[0], var, dec))
-        if rec:
-            hw_flops = rec["fp32_flops_per_launch"]
-    except (OSError, ValueError, KeyError):
-        hw_flops = None
-    ref_achieved = achieved
-    if hw_flops:
-        achieved = hw_flops / (kern_ms * 1e-3) / 1e12
+    # what the hardware issued and moved per evaluation of this workload (rocprofv3
+    # SQ_INSTS_VALU_FLOPS_FP32 x 64 lanes; FETCH_SIZE and WRITE_SIZE scaled by the same
+    # counters on a copy of known size): null where no profile of these kernels is recorded
+    key = workload_name(args, pos.shape[0], var, dec)
+    rec = profiled(os.path.join(ROOT, "profiles", "traffic.json"), key, npairs)
+    traffic = rec and rec["bytes_per_launch"]
+    rec = profiled(os.path.join(ROOT, "profiles", "valu_flops.json"), key, npairs)
+    hw_flops = rec and rec["fp32_flops_per_launch"]
+    achieved = hw_flops and hw_flops / (kern_ms * 1e-3) / 1e12
+    log("kernel sources %s  pairs %d" % (kernel_sources(), npairs))
 
     cpu = None
     if not args.no_cpu:
@@ -245,14 +256,13 @@ def main():
                    "mean_group": st["mean_group"], "decomposition": dec,
                    "host_build_s": st["t_tree"] + st["t_lists"]},
         "roofline": {"bound": "valu", "achieved": achieved, "peak": PEAK_FP32_TFLOPS,
-                     "unit": "TFLOP/s", "frac": achieved / PEAK_FP32_TFLOPS, "traffic": traffic,
+                     "unit": "TFLOP/s", "frac": achieved and achieved / PEAK_FP32_TFLOPS,
+                     "traffic": traffic,
                      "kernel_ms": kern_ms, "algorithmic_bytes": nbytes,
                      "hbm_GBs_algorithmic": nbytes / (kern_ms * 1e-3) / 1e9,
-                     "counted": "hardware" if hw_flops else "reference",
                      "reference_achieved": ref_achieved,
-                     "hw_fp32_flops_per_launch": hw_flops,
-                     "hw_frac": achieved / PEAK_FP32_TFLOPS if hw_flops else None},
-        "pct_fp32_peak": 100.0 * achieved / PEAK_FP32_TFLOPS,
+                     "hw_fp32_flops_per_launch": hw_flops},
+        "pct_fp32_peak": achieved and 100.0 * achieved / PEAK_FP32_TFLOPS,
         "errors": errors,
         "baselines": baselines,
         "cpu_baseline": cpu,

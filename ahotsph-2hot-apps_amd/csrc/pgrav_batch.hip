@@ -956,7 +956,8 @@ hipError_t launch_batch(const BatchView &v, int variant, int persistent_blocks, 
         if (e != hipSuccess)
             return e;
     }
-    A.lw = split_log2(v.ngroups, v.wave_slots);
+    A.lw = v.periodic == 1 ? split_log2_ewald(v.ngroups, v.wave_slots, variant == VAR_F64)
+                           : split_log2(v.ngroups, v.wave_slots);
     A.given = 0;
     A.cus = v.wave_slots / 32;
     if (persistent_blocks < 0)

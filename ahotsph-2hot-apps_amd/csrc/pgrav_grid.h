@@ -31,6 +31,29 @@ constexpr int split_log2(int ngroups, int wave_slots) {
     return ngroups < 4 * wave_slots ? 3 : 2;
 }
 
+// The same for the Ewald kernels, whose waves take 6 KB (FP64 12 KB) of LDS: 24 (12) a CU in
+// any split, and a workgroup's leave their places to nobody until its last is done.  us per
+// evaluation by 1, 2, 4, 8 waves a group, passes of three plans in turn on three streams /
+// one plan alone; in brackets one wave a group, square roots and divides, every cell in pairs:
+//   4,098 (lattice 64^3)     1555/1466  1437/1338  1390/1228  1413/1221  [1537/2013]
+//   7,878 (68^3)             2522/3051  2471/2674  2455/2424  2573/2420  [2559/2993]
+//   8,435 (73^3)             2650/3118  2638/2742  2676/2564  2742/2589  [2713/3249]
+//   11,065 (80^3)            2731/3173  2767/2816  2764/2651  2874/2696  [2785/3224]
+//   14,045 (88^3)            4552/5660  4637/4889  4628/4585  4752/4653  [4531/5645]
+//   16,384 (96^3)            3312/3588  3288/3307  3387/3220  4100/3351  [3458/3964]
+//   32,767 (112^3)           3741/4244  3816/3939  3933/3973  5247/4507  [5013/5603]
+//   FP64 4,098               2799/3459  2804/2892  2838/2755             [2862/3486]
+//   FP64 11,065              6488/7126  6664/6674  6853/6584             [6389/7392]
+//   FP64 16,384              8631/8576  8983/8457  9278/8484             [8836/9382]
+//   FP64 32,767            11984/11151 12369/11281 12253/11009          [12861/13406]
+constexpr int split_log2_ewald(int ngroups, int wave_slots, bool fp64) {
+    if (ngroups < wave_slots * 3 / 4)
+        return 3;
+    if (fp64 || ngroups > (1 << 25) - NXCD)
+        return 0;
+    return ngroups < wave_slots * 5 / 4 ? 2 : 1;
+}
+
 // Workgroups of a persistent launch, `waves` waves each: as many as asked for, but no more
 // than there are groups, or (negative) those of -blocks waves; a multiple of NXCD, because
 // every XCD needs workgroups to drain its slice.  (Counted in waves, a grid of 256 was 32

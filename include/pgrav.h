@@ -155,8 +155,8 @@ typedef struct {
                               (groups are body sets, read through a slot table) */
     int persistent_blocks; /* 0: one workgroup per group; >0: persistent grid of that many
                               workgroups (no more than groups, rounded up to a multiple of 8),
-                              each of the 4 to 16 waves that share a group's lists (fewer
-                              from ~2^24 groups on); -1 (default): 32 waves per CU */
+                              each of the 1 to 16 waves that share a group's lists
+                              (by the number of groups); -1 (default): 32 waves per CU */
     int fp64;              /* also build the FP64 tables (variants 3 and 4) */
     int dispatch;          /* 0: global longest-first; per-XCD Morton slices of equal estimated
                               cost, ordered inside 1: longest-first, 2 (default): Morton order,

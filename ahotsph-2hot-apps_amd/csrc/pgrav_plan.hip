@@ -19,6 +19,7 @@
 #include "pgrav_batch.h"
 #include "pgrav_device.h"
 #include "pgrav_ewald.h"
+#include "pgrav_far.h"
 #include "pgrav_host.h"
 #include "pgrav_le.h"
 #include "pgrav_le_launch.h"
@@ -187,13 +188,14 @@ static int device_wave_slots() {
 //   order 0, 1 M (26,465, 813)        821  858    tolerance 1 M (16,454, 47 + 22 + 1,704) 1220 1204
 //   Ewald 64^3 (4,102, 794)          1204 1260    Ewald 96^3 (16,384, 794) 3482 3247
 //   Ewald 128^3 (32,795, 910)        5012 3847
-// The line is on the safe side at clustered 131,072 and at order 2, and blind to what it
-// does not look at, the cells' distances: with softening none nearer than 100 eps is far,
-// and where that leaves none the scan of the lists is lost (clustered 1 M by eps: 1e-4 1821,
-// 1e-3 2095, 1e-2 2831 against 2596 in pairs; Plummer 262,144 at eps 0.1 906 against 868).
+// The line is on the safe side at clustered 131,072 and at order 2.  It says nothing of the
+// cells' distances, and softened plans have no far cell nearer than 100 eps: below a fifth
+// of the listed work far, in 64 groups of the plan, the scan of the lists costs more than it
+// saves (clustered by eps, share: 1 M 3e-4 0.65 1877, 1e-3 0.50 2095, 3e-3 0.22 2508, 1e-2
+// 0.004 2831 against 2596 in pairs; 262,144 3e-3 0.29 609, 1e-2 0.005 677 against 619).
 // Groups of one body have no expansion and leave k_far at once; where all are (400,000
 // bodies), 22.3 ms a pass without it and 22.6 with it.
-static bool far_pays(const Lists &L, int wave_slots, int periodic) {
+static bool far_pays(const Tree &t, const Lists &L, const pgrav_params &prm, int wave_slots) {
     int64_t G = 0, hexa = 0, quad = 0;
     for (int64_t g = 0; g < L.ngroups; g++)
         if (L.gcount[g] > 1) {
@@ -201,8 +203,43 @@ static bool far_pays(const Lists &L, int wave_slots, int periodic) {
             hexa += L.off[L_HEXA][g + 1] - L.off[L_HEXA][g];
             quad += L.off[L_QUAD][g + 1] - L.off[L_QUAD][g];
         }
-    return 38 * hexa + 8 * quad > 6500 * G + (int64_t)4000 * wave_slots &&
-           (periodic != 1 || G >= 2 * (int64_t)wave_slots);
+    if (38 * hexa + 8 * quad <= 6500 * G + (int64_t)4000 * wave_slots ||
+        (prm.periodic == 1 && G < 2 * (int64_t)wave_slots))
+        return false;
+    int64_t far = 0, all = 0;
+    const int S = 64, f = 2 * prm.nimage + 1;
+    for (int s = 0; s < S; s++) {
+        const int64_t g = L.ngroups * s / S;
+        const double *c = &L.gcenter[4 * g];
+        double rs2 = 0;
+        for (int k = 0; k < L.gcount[g]; k++) {
+            const int64_t i = L.gslots.empty() ? L.gfirst[g] + k : L.gslots[L.gslot_off[g] + k];
+            double r2 = 0;
+            for (int q = 0; q < 3; q++) r2 += (t.pos[3 * i + q] - c[q]) * (t.pos[3 * i + q] - c[q]);
+            rs2 = std::max(rs2, r2);
+        }
+        const double far2 = std::max(rs2 / (FAR_RHO * FAR_RHO),
+                                     prm.soft_type == SOFT_PLUMMER ? prm.eps * prm.eps / FAR_ETA : 0.0);
+        for (int kind : {L_HEXA, L_QUAD})
+            for (int64_t at = L.off[kind][g]; at < L.off[kind][g + 1]; at++) {
+                const double *X = &t.cofm[3 * (size_t)L.idx[kind][at]];
+                const int im = prm.periodic == 2 ? L.img[kind][at] : 0;
+                const int shift[3] = {im / (f * f), (im / f) % f, im % f};
+                double r2 = 0;
+                for (int q = 0; q < 3; q++) {
+                    double d = X[q] - c[q];
+                    if (prm.periodic == 1)
+                        d -= prm.box * rint(d / prm.box);
+                    else if (prm.periodic == 2)
+                        d += prm.box * (shift[q] - prm.nimage);
+                    r2 += d * d;
+                }
+                const int w = kind == L_HEXA ? 38 : 8;
+                all += w;
+                far += rs2 > 0 && r2 > far2 ? w : 0;
+            }
+    }
+    return 5 * far >= all;
 }
 
 static hipStream_t stream_of(Plan *P, void *stream) {
@@ -429,6 +466,7 @@ void *pgrav_plan_create(const double *pos3, const double *mass, int64_t n, const
         Lists &L = P->lists;
         P->v.ngroups = (int)L.ngroups;
         P->v.wave_slots = device_wave_slots();
+        const bool expand = far_pays(P->tree, L, *p, P->v.wave_slots);  // (reads the lists' host copy)
         P->v.gfirst = P->upload(L.gfirst.data(), L.gfirst.size());
         P->v.gcount = P->upload(L.gcount.data(), L.gcount.size());
         if (!L.gslots.empty()) {
@@ -509,7 +547,7 @@ void *pgrav_plan_create(const double *pos3, const double *mass, int64_t n, const
             P->v.ewald32 = t32;
             P->v.ewald64 = t64;
         }
-        if (far_pays(L, P->v.wave_slots, p->periodic))
+        if (expand)
             P->far_alloc(L.off[L_HEXA].back() + L.off[L_QUAD].back() + L.off[L_MONO].back());
         if (!check(hipStreamSynchronize(P->stream), "hipStreamSynchronize"))
             throw std::runtime_error("sync");

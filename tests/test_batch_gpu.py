@@ -418,23 +418,31 @@ def test_far_cells_of_a_vanishing_group(gpu_lib, size):
     plan.close()
 
 
-@pytest.mark.parametrize("gmax,expands", [(1, False), (8, True)])
-def test_groups_of_one_body_have_no_expansions(gpu_lib, gmax, expands):
-    """Seen by the memory a plan takes: the expansions' workspace repeats the cell lists."""
+def test_plans_that_expansions_do_not_pay_for(gpu_lib):
+    """Groups of one body have no expansion, and a softening of the system's size no far
+    cell (none is nearer than 100 eps).  Seen by the memory a plan takes: the expansions'
+    workspace repeats the cell lists."""
     import torch
     from pgrav import batch, ics
     pos, mass = ics.clustered(80000, seed=21, nhalo=24)
-    kw = dict(theta=0.4, order=4, eps=1e-3, group_max=gmax, leaf_max=16, merge_groups=0, fp64=False)
+    kw = dict(theta=0.4, order=4, leaf_max=16, merge_groups=0, fp64=False)
+
+    def took(gmax, eps):
+        free = torch.cuda.mem_get_info()[0]
+        plan = batch.Plan(pos, mass, group_max=gmax, eps=eps, **kw)
+        used, st = free - torch.cuda.mem_get_info()[0], plan.stats()
+        plan.close()
+        return used, st
     batch.Plan(pos[:1000], mass[:1000], **kw).close()  # the library's own start-up
-    free = torch.cuda.mem_get_info()[0]
-    plan = batch.Plan(pos, mass, **kw)
-    took = free - torch.cuda.mem_get_info()[0]
-    st = plan.stats()
-    plan.close()
-    cells = 4 * sum(st["entries_" + k] for k in ("hexa", "quad", "mono"))
-    base = 4 * st["entries_body"] + cells + 48 * st["n"] + 96 * st["ngroups"] + 256 * st["nnodes"]
-    assert cells > 2 ** 25, cells  # well above an allocation's granularity
-    assert (took > base + 0.6 * cells) == expands, (took, base, cells)
+    whole, st = took(8, 1e-3)
+    lists = 4 * sum(st["entries_" + k] for k in ("hexa", "quad", "mono"))
+    less, _ = took(8, 0.03)  # the same lists
+    # (each allocation takes whole units of 2 MB)
+    assert abs(whole - less - lists - 32 * st["n"]) < 16 * 2 ** 20, (whole, less, lists)
+    one, st = took(1, 1e-3)
+    lists = 4 * sum(st["entries_" + k] for k in ("hexa", "quad", "mono"))
+    base = 4 * st["entries_body"] + lists + 48 * st["n"] + 96 * st["ngroups"] + 256 * st["nnodes"]
+    assert one < base + 0.5 * lists, (one, base, lists)
 
 
 def test_results_stay_whole_under_the_next_evaluation(gpu_lib):

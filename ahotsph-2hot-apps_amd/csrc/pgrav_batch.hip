@@ -10,8 +10,8 @@
 //                          order-0 cells, bodies (u32 node / sorted-body slots)
 //   lpt    int[G]          groups by decreasing cost (longest first)
 //
-// Execution: one lane per sink (groups hold <= 64), 4 to 16 wave64s per group, each
-// with an equal run of every list kind (split_log2); their sums meet in LDS.
+// Execution: one lane per sink (groups hold <= 64), 1 to 16 wave64s per group, each
+// with an equal run of every list kind (pgrav_grid.h); their sums meet in LDS.
 // A list is consumed in tiles of 64 entries: each lane fetches one entry's FP64
 // centre, subtracts the FP64 group centre, rounds the small offset to FP32 and
 // parks it in LDS; then every lane sweeps the tile, reading the offset as an

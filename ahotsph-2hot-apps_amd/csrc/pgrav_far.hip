@@ -12,7 +12,7 @@
 //
 // Bound by VALU at two waves per SIMD: 1,500 instructions per 64 order-4 cells (1,050
 // order 2, 345 order 0) against 110 (45, 16) x 64 in pairs, ~110 per 64 entries scanned
-// and ~2,300 per group.  Clustered 16.8 M: 7.3 ms, which take 62 % of the order-4 cells
+// and ~2,300 per group.  Clustered 16.8 M: 7.0 ms, which take 62 % of the order-4 cells
 // out of the pair kernel, 42.5 -> 20 ms.
 #include <math.h>
 

@@ -292,7 +292,8 @@ def test_shared_lists_match_oracle(setup, n):
 
 
 def _far_pays(st, ewald):
-    # the rule of pgrav_plan.hip for 256 CUs (the Ewald kernel's too)
+    # the rule of pgrav_plan.hip for 256 CUs (the Ewald kernel's too), by the lists' lengths;
+    # of the work listed by the plans here 0.3 and more is far, where the rule asks for 0.2
     return 38 * st["entries_hexa"] + 8 * st["entries_quad"] > 6500 * st["ngroups"] + 4000 * 8192 \
         and (not ewald or st["ngroups"] >= 2 * 8192)
 
